@@ -319,15 +319,18 @@ extern "C" int rfsn_blockwise_attention(const void* q, int32_t B, int32_t Hq, in
   RFSN_REQUIRE(stride_t % 8 == 0 && stride_h % 8 == 0, "blockwise_attention: K/V rows must be 16-byte aligned");
   const int G = Hq / Hkv;
   hipStream_t s = (hipStream_t)stream;
+  const float sl2 = scale * kLog2e;
+  RFSN_REQUIRE(ws && ws_bytes >= rfsn_attention_workspace_bytes(B, Hq, D, 1),
+               "blockwise_attention: workspace too small");
+  if (G != 1 && G != 2 && G != 4 && G != 8)
+    return fail(RFSN_ERR_UNSUPPORTED, "blockwise_attention: Hq/Hkv must be 1, 2, 4 or 8");
+  if (prompt_attention_ok(q, B, Hq, Hkv, D, k, v, T, sl2, out, ws))
+    return launch_prompt_attention(q, B, Hq, Hkv, D, k, v, T, stride_t, stride_h, sl2, causal, qpos, out, ws, ws_bytes,
+                                   s);
   int splits = T > 0 ? choose_splits(T, (int64_t)B * Hkv) : 1;
-  if (ws_bytes < rfsn_attention_workspace_bytes(B, Hq, D, splits)) {
-    splits = 1;
-    RFSN_REQUIRE(ws && ws_bytes >= rfsn_attention_workspace_bytes(B, Hq, D, 1),
-                 "blockwise_attention: workspace too small");
-  }
+  if (ws_bytes < rfsn_attention_workspace_bytes(B, Hq, D, splits)) splits = 1;
   const int64_t tps = T > 0 ? ceil_div(ceil_div(T, splits), 64) * 64 : 64;
   dim3 grid((unsigned)splits, (unsigned)Hkv, (unsigned)B);
-  const float sl2 = scale * 1.4426950408889634f;
   // the batch axis of q/out is separate; K/V are shared by the batch of queries
   // (attention.py:48: q [B,H,D] are queries over one cache)
 #define RFSN_EXACT(DD, GG)                                                                                       \

@@ -1,0 +1,75 @@
+"""Many-query exact attention on the matrix cores against float64.
+
+The kernel takes 64, 128 or 256 query rows per block, 64-token tiles and one or
+more token splits; the shapes sit at those edges.  Tolerance: the fp16 result's
+rounding (2^-11 of the value) plus fp32 sums of weights kept to 22 bits, so
+2^-11 |out| + 2^-15 max|v| (2^-22 per weight and 2^-24 per product would be
+far below the second term; it covers the exponent of a score of up to 64)."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(q, k, v, scale, pos):
+    B, Hq, D = q.shape
+    T, Hkv, _ = k.shape
+    G = Hq // Hkv
+    kk, vv = k.astype(np.float64), v.astype(np.float64)
+    out = np.zeros((B, Hq, D))
+    for h in range(Hq):
+        s = q[:, h].astype(np.float64) @ kk[:, h // G].T * scale
+        if pos is not None:
+            s = np.where(np.arange(T)[None] <= pos[:, h, None], s, -np.inf)
+        m = s.max(1, keepdims=True)
+        w = np.where(np.isfinite(s), np.exp(s - np.where(np.isfinite(m), m, 0)), 0)
+        n = w.sum(1, keepdims=True)
+        out[:, h] = (w @ vv[:, h // G]) / np.where(n > 0, n, 1)
+    return out
+
+
+CASES = [  # B, Hq, Hkv, T, D
+    (4, 2, 2, 1, 64), (5, 8, 4, 63, 64), (33, 4, 2, 64, 128), (16, 8, 2, 65, 64), (64, 2, 2, 129, 128),
+    (65, 2, 2, 1537, 128), (150, 4, 2, 1600, 64), (257, 4, 4, 2000, 64), (600, 4, 2, 6200, 64), (7, 8, 1, 5000, 64),
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,D", CASES)
+@pytest.mark.parametrize("mode", ["full", "causal", "mixed"])
+def test_prompt_attention(device, B, Hq, Hkv, T, D, mode):
+    import torch
+    from apple_amd import kernels as K
+
+    g = np.random.default_rng(B * 1000 + T)
+    q, k, v = (g.standard_normal(s, dtype=np.float32).astype(np.float16)
+               for s in ((B, Hq, D), (T, Hkv, D), (T, Hkv, D)))
+    q[B // 2] *= np.float16(8)  # one sharp query
+    if mode == "full":
+        pos = None
+    elif mode == "causal":
+        pos = np.repeat((np.arange(B) + T - B)[:, None], Hq, 1).astype(np.int32)  # negative: nothing allowed
+    else:
+        pos = g.integers(-2, T + 2, (B, Hq)).astype(np.int32)
+    dev = lambda a: torch.from_numpy(a).to(device)
+    got = K.blockwise_attention(dev(q), dev(k), dev(v), D ** -0.5, pos is not None,
+                                None if pos is None else dev(pos)).double().cpu().numpy()
+    want = _ref(q, k, v, D ** -0.5, pos)
+    assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + np.abs(v).max().astype(np.float64) * 2.0 ** -15)
+    if pos is not None:
+        assert not got[pos < 0].any()
+
+
+def test_prompt_attention_strides_and_views(device):
+    """Strided K/V rows (a head-major ring), and a query view off 16-byte alignment (the scalar kernel's)."""
+    import torch
+    from apple_amd import kernels as K
+
+    g = torch.Generator().manual_seed(5)
+    ring = torch.randn(2, 3, 200, 64, generator=g).half().to(device)  # [K/V][head][token][D]
+    k, v = (ring[i].permute(1, 0, 2)[7:190] for i in range(2))
+    q = torch.randn(9 * 3 * 64 + 1, generator=g).half().to(device)
+    want = _ref(q[1:].view(9, 3, 64).cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), 0.125, None)
+    for qq in (q[1:].view(9, 3, 64), q[1:].view(9, 3, 64).clone()):
+        got = K.blockwise_attention(qq, k, v, 0.125, False, None).double().cpu().numpy()
+        assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + 5 * 2.0 ** -15)
