@@ -14,6 +14,28 @@
 namespace rfsn {
 namespace {
 
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float float8v __attribute__((ext_vector_type(8)));
+
+// Coordinates 8g .. 8g + 7 of the vector whose codes are at code: one centroid
+// slice (d a multiple of 8) or two centroids (d = 4) of the [M][C][d] codebooks.
+template <int d>
+__device__ __forceinline__ half8 centroid8(const uint8_t* __restrict__ code, uint32_t g, int C,
+                                           const uint16_t* __restrict__ cb) {
+  if constexpr (d == 4) {
+    const uint32_t c = *reinterpret_cast<const uint16_t*>(code + 2 * g);
+    const uint32_t c0 = min(c & 0xFF, (uint32_t)C - 1), c1 = min(c >> 8, (uint32_t)C - 1);
+    const half4 a = *reinterpret_cast<const half4*>(cb + ((2 * g) * C + c0) * 4);
+    const half4 b = *reinterpret_cast<const half4*>(cb + ((2 * g + 1) * C + c1) * 4);
+    return half8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  } else {
+    const uint32_t m = g / (d / 8);
+    const uint32_t c = min((uint32_t)code[m], (uint32_t)C - 1);
+    return *reinterpret_cast<const half8*>(cb + (m * C + c) * d + (g % (d / 8)) * 8);
+  }
+}
+
 // One thread per (vector, group of 4 coordinates).
 __global__ void __launch_bounds__(256)
 decode_ext_kernel(int64_t n, int D, const uint8_t* __restrict__ pq, int M, int C, const uint16_t* __restrict__ pq_cb,
@@ -47,6 +69,41 @@ decode_ext_kernel(int64_t n, int D, const uint8_t* __restrict__ pq, int M, int C
   uint16_t* o = out + v * ldo + i0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = r[e];
+}
+
+// The same for the formats in use: 8 coordinates per thread, so a row leaves in
+// 16-byte stores and a centroid arrives in one 8- or 16-byte load.  d = the
+// subspace size of both stages (4, or a multiple of 8); SPARSE: k = 4, with the
+// indices of a row as one word; 1 << shift = D / 8 threads per row.  Bound: the
+// codebook gathers (64 KB of codebooks over a 32 KB L1), then the row stores.
+// 8,191 x 8 vectors, M 16 + RVQ 16 + top-4: 27.4 us with the kernel above (2-byte
+// accesses, a division per coordinate), 9.4 us here.
+template <int d, bool RVQ, bool SPARSE>
+__global__ void __launch_bounds__(256)
+decode_ext8_kernel(int64_t n, int shift, const uint8_t* __restrict__ pq, int M, int C, const uint16_t* __restrict__ pq_cb,
+                   const uint8_t* __restrict__ rvq, int Cr, const uint16_t* __restrict__ rvq_cb,
+                   const uint8_t* __restrict__ sidx, const uint16_t* __restrict__ sval, int add_zero,
+                   uint16_t* __restrict__ out, int64_t ldo) {
+  const int64_t v = ((int64_t)blockIdx.x << (8 - shift)) + (threadIdx.x >> shift);
+  const uint32_t g = threadIdx.x & ((1u << shift) - 1);
+  if (v >= n) return;
+  half8 r = centroid8<d>(pq + v * M, g, C, pq_cb);
+  if constexpr (RVQ) {
+    r = r + centroid8<d>(rvq + v * M, g, Cr, rvq_cb);
+  } else if (add_zero) {
+    r = r + (half8)(_Float16)0.f;
+  }
+  if constexpr (SPARSE) {
+    const uint32_t ix = reinterpret_cast<const uint32_t*>(sidx)[v];
+    const half4 val = __builtin_bit_cast(half4, reinterpret_cast<const uint2*>(sval)[v]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t at = ((ix >> (8 * j)) & 0xFF) - g * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = at == (uint32_t)e ? (_Float16)(r[e] + val[j]) : r[e];
+    }
+  }
+  *reinterpret_cast<half8*>(out + v * ldo + g * 8) = r;
 }
 
 // One thread per sparse entry (vector v, slot j): the corrected coordinate
@@ -225,6 +282,76 @@ decode_ref_corr_kernel(int64_t n, int64_t active, int D, const uint8_t* __restri
   out[v * D + i] = hadd_bits(pq_cb[((size_t)m * C + min((int)pq[v * M + m], C - 1)) * d + (i - m * d)], corr);
 }
 
+// The two kernels above with 8 coordinates per thread (d a multiple of 8, so a
+// thread lies in one PQ subspace): 16-byte codeword, centroid and row accesses,
+// and the codewords of four layers requested together.  Row r is left to the
+// correction kernel where its index is known without a search, offsets[r] = r
+// (every row of a store whose rows are all active), and then written once.
+// Bound: the L codeword rows per vector (L2 / MALL), then the row stores.
+// 131,072 rows of D 128, 4 layers of 4,096, all active: 42 + 116 us with one
+// thread per coordinate, 1.9 + 17.8 us here.
+//
+// Base rows: a wave looks at 64 rows' offsets at once, then writes those that
+// need it, 64 >> shift rows at a time (1 << shift = D / 8 threads per row).
+template <int d>
+__global__ void __launch_bounds__(256)
+decode_ref_base8_kernel(int64_t n, int shift, const uint8_t* __restrict__ pq, int M, int C,
+                        const uint16_t* __restrict__ pq_cb, const int32_t* __restrict__ offsets, int64_t active,
+                        uint16_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63u);
+  const int64_t r = row0 + lane;
+  const uint64_t todo = __ballot(r < n && !(r < active && offsets[r] == r));
+  if (todo == 0) return;
+  const uint32_t g = lane & ((1u << shift) - 1);
+  for (int i = lane >> shift; i < 64; i += 64 >> shift) {
+    if (!((todo >> i) & 1)) continue;
+    const int64_t v = row0 + i;
+    *reinterpret_cast<half8*>(out + ((v << shift) + g) * 8) =
+        centroid8<d>(pq + v * M, g, C, pq_cb) + (half8)(_Float16)0.f;
+  }
+}
+
+template <int d>
+__global__ void __launch_bounds__(256)
+decode_ref_corr8_kernel(int64_t n, int64_t active, int shift, const uint8_t* __restrict__ pq, int M, int C,
+                        const uint16_t* __restrict__ pq_cb, const uint16_t* __restrict__ codes,
+                        const int32_t* __restrict__ offsets, int L, int Cr, const uint16_t* __restrict__ rvq_cb,
+                        uint16_t* __restrict__ out) {
+  const int D = 8 << shift;
+  const int64_t a = ((int64_t)blockIdx.x << (8 - shift)) + (threadIdx.x >> shift);
+  const uint32_t g = threadIdx.x & ((1u << shift) - 1);
+  if (a >= active) return;
+  const int64_t v = offsets[a];
+  if (v < 0 || v >= n) return;  // offsets outside the decoded rows are ignored
+  const half8 base = centroid8<d>(pq + v * M, g, C, pq_cb);
+  const uint16_t* code = codes + a * L;
+  const bool wide = L % 4 == 0 && ((uintptr_t)codes & 7) == 0;
+  float8v total = (float8v)0.f;
+  int l = 0;
+  for (; l + 4 <= L; l += 4) {
+    uint16_t c[4];
+    if (wide) {
+      const uint2 w2 = *reinterpret_cast<const uint2*>(code + l);
+      c[0] = (uint16_t)w2.x, c[1] = (uint16_t)(w2.x >> 16), c[2] = (uint16_t)w2.y, c[3] = (uint16_t)(w2.y >> 16);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = code[l + u];
+    }
+    half8 w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      w[u] = *reinterpret_cast<const half8*>(rvq_cb + ((size_t)(l + u) * Cr + min((int)c[u], Cr - 1)) * D + g * 8);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) total += __builtin_convertvector(w[u], float8v);
+  }
+  for (; l < L; ++l)
+    total += __builtin_convertvector(
+        *reinterpret_cast<const half8*>(rvq_cb + ((size_t)l * Cr + min((int)code[l], Cr - 1)) * D + g * 8), float8v);
+  const half8 corr = __builtin_convertvector(total, half8);
+  *reinterpret_cast<half8*>(out + v * D + g * 8) = base + corr;
+}
+
 // k-means: per-(subspace, centroid) sums in float64 via atomics, then mean.
 __global__ void kmeans_accum_kernel(const uint16_t* __restrict__ x, int64_t n, int D, int64_t ldx,
                                     const uint8_t* __restrict__ codes, int M, int C, double* __restrict__ sums,
@@ -348,6 +475,45 @@ extern "C" int rfsn_decode(const rfsn_format* f, const rfsn_codes* codes, int64_
   RFSN_REQUIRE(f->sparse_k == 0 || (codes->sparse_idx && codes->sparse_val), "decode: sparse stage needs codes");
   RFSN_REQUIRE(ldo >= f->head_dim, "decode: bad leading dimension");
   if (n == 0) return RFSN_OK;
+  // 8 coordinates per thread where both stages share a subspace size of 4 or a
+  // multiple of 8, the sparse stage is absent or top-4, and every row is
+  // aligned for the wide accesses; the general kernel otherwise
+  const int D = f->head_dim, d = D / f->pq_subspaces, k = f->sparse_k;
+  auto aligned = [](const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; };
+  const uintptr_t ca = d == 4 ? 2 : 1, cba = d == 4 ? 8 : 16;
+  const bool has_rvq = f->rvq_subspaces > 0;
+  if (D >= 8 && D <= 512 && (D & (D - 1)) == 0 && (d == 4 || d == 8 || d == 16 || d == 32) && (!has_rvq || f->rvq_subspaces == f->pq_subspaces) &&
+      (k == 0 || k == 4) && ldo % 8 == 0 && aligned(out, 16) && aligned(codes->pq, ca) && aligned(pq_cb, cba) &&
+      (!has_rvq || (aligned(codes->rvq, ca) && aligned(rvq_cb, cba))) &&
+      (k == 0 || (aligned(codes->sparse_idx, 4) && aligned(codes->sparse_val, 8)))) {
+    const int shift = __builtin_ctz(D / 8);
+    const dim3 grid((unsigned)ceil_div(n << shift, 256));
+#define RFSN_DECODE(d_, r_, s_)                                                                                       \
+  hipLaunchKernelGGL((decode_ext8_kernel<d_, r_, s_>), grid, dim3(256), 0, (hipStream_t)stream, n, shift, codes->pq,  \
+                     f->pq_subspaces, f->pq_centroids, (const uint16_t*)pq_cb, codes->rvq, f->rvq_centroids,          \
+                     (const uint16_t*)rvq_cb, codes->sparse_idx, (const uint16_t*)codes->sparse_val, add_zero,        \
+                     (uint16_t*)out, ldo)
+#define RFSN_DECODE_D(d_)                                  \
+  if (has_rvq) {                                           \
+    if (k) RFSN_DECODE(d_, true, true);                    \
+    else RFSN_DECODE(d_, true, false);                     \
+  } else {                                                 \
+    if (k) RFSN_DECODE(d_, false, true);                   \
+    else RFSN_DECODE(d_, false, false);                    \
+  }
+    if (d == 4) {
+      RFSN_DECODE_D(4)
+    } else if (d == 8) {
+      RFSN_DECODE_D(8)
+    } else if (d == 16) {
+      RFSN_DECODE_D(16)
+    } else {
+      RFSN_DECODE_D(32)
+    }
+#undef RFSN_DECODE_D
+#undef RFSN_DECODE
+    return check_launch("decode");
+  }
   const int64_t total = n * (f->head_dim / 4);
   hipLaunchKernelGGL(decode_ext_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, (hipStream_t)stream, n,
                      f->head_dim, codes->pq, f->pq_subspaces, f->pq_centroids, (const uint16_t*)pq_cb, codes->rvq,
@@ -435,6 +601,30 @@ extern "C" int rfsn_decode_ref(const uint8_t* pq, int64_t n, int32_t D, int32_t 
   RFSN_REQUIRE(pq && pq_cb && out && D > 0 && M > 0 && D % M == 0, "decode_ref: bad arguments");
   RFSN_REQUIRE(active == 0 || (rvq_codes && offsets && rvq_cb && L >= 1), "decode_ref: RVQ arguments missing");
   hipStream_t s = (hipStream_t)stream;
+  // 8 coordinates per thread where a thread then lies in one subspace and the
+  // rows are aligned for 16-byte accesses; the general kernels otherwise
+  const int d = D / M;
+  auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  if (D <= 512 && (D & (D - 1)) == 0 && (d == 8 || d == 16 || d == 32) && aligned(pq_cb) && aligned(out) && (active == 0 || aligned(rvq_cb))) {
+    const int shift = __builtin_ctz(D / 8);
+#define RFSN_DECODE_REF(d_)                                                                                           \
+  if (n > 0)                                                                                                          \
+    hipLaunchKernelGGL(decode_ref_base8_kernel<d_>, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, n, shift, pq,  \
+                       M, C, (const uint16_t*)pq_cb, offsets, active, (uint16_t*)out);                                \
+  if (active > 0)                                                                                                     \
+    hipLaunchKernelGGL(decode_ref_corr8_kernel<d_>, dim3((unsigned)ceil_div(active << shift, 256)), dim3(256), 0, s,  \
+                       n, active, shift, pq, M, C, (const uint16_t*)pq_cb, rvq_codes, offsets, L, Cr,                 \
+                       (const uint16_t*)rvq_cb, (uint16_t*)out)
+    if (d == 8) {
+      RFSN_DECODE_REF(8);
+    } else if (d == 16) {
+      RFSN_DECODE_REF(16);
+    } else {
+      RFSN_DECODE_REF(32);
+    }
+#undef RFSN_DECODE_REF
+    return check_launch("decode_ref");
+  }
   if (n > 0) {
     hipLaunchKernelGGL(decode_ref_base_kernel, dim3((unsigned)ceil_div(n * D, 256)), dim3(256), 0, s, n, D, pq, M, C,
                        (const uint16_t*)pq_cb, (uint16_t*)out);
