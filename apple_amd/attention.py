@@ -8,9 +8,9 @@ values may have fewer heads than the query (GQA): query head ``h`` reads KV
 head ``h // (Hq // Hkv)`` (llama32_adapter.py:384-386).
 ``RFSNHybridAttentionMLX`` attends the two compressed stores in one launch
 of the decode-in-register kernel (``kernels.ref_attention``), which rebuilds
-each K/V vector in registers with the decode's rounding (attention.py:159-171
-decodes both stores, then attends); stores outside that kernel's shapes are
-decoded and attended as the reference does.  The tiled fused
+each K/V vector in registers with the decode's rounding; many queries
+(``kernels.decode_first``) and stores outside that kernel's shapes decode both
+stores, then attend, as the reference does (attention.py:159-171).  The tiled fused
 dequant-attention kernel is driven by the cache (``cache.py``), which owns the
 code layout that kernel streams.
 """
@@ -103,7 +103,8 @@ class RFSNHybridAttentionMLX:
     def _fused(self, q, key_store, value_store, quantizer, causal, query_positions) -> torch.Tensor:
         """Decode-and-attend in one kernel: each K/V vector is rebuilt in
         registers with the reference's rounding (quantization.py:310-319) and
-        never written to HBM (rfsn_ref_attention)."""
+        never written to HBM (rfsn_ref_attention).  Many queries share one
+        decode of the window instead (``kernels.decode_first``)."""
         B, Hq, _ = q.shape
         T = key_store.num_tokens
         if T == 0:
@@ -119,8 +120,14 @@ class RFSNHybridAttentionMLX:
         # tokens for the tables to beat the exact decode
         tol = quantizer.config.score_table_tolerance
         tables = {}
-        if (tol is not None and not quantizer.subspace and B * Hq <= REF_TABLES_MAX_QUERY_HEADS
-                and T >= K.ref_tables_min_tokens(Hq // key_store.num_heads, B)):
+        use_tables = (tol is not None and not quantizer.subspace and B * Hq <= REF_TABLES_MAX_QUERY_HEADS
+                      and T >= K.ref_tables_min_tokens(Hq // key_store.num_heads, B))
+        if K.decode_first(B, Hq, key_store.num_heads, int(q.shape[-1]), T, use_tables):
+            # a chunk of a prompt: rebuild each vector once, then attend on the matrix cores
+            out = K.blockwise_attention(q.to(device=dev, dtype=torch.float16), _decode_compressed_tensor(kst, quantizer),
+                                        _decode_compressed_tensor(vst, quantizer), self.scale, causal, pos)
+            return out.to(q.dtype)
+        if use_tables:
             tables = dict(score_tables=float(tol), table_stats=self._table_stats(quantizer))
         # the tables read a head's codes in whole lines from a head-major
         # copy, kept per store (only for stores already on the device, which

@@ -863,6 +863,30 @@ def ref_tables_min_tokens(group: int, queries: int = 1) -> int:
     return base * (q + 1) // (2 * q)
 
 
+def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, tokens: int, tables: bool) -> bool:
+    """Whether ``queries`` query tokens over ``tokens`` coded ones are faster
+    as decode-once-then-attend (``decode_ref`` / ``decode``, then the matrix
+    cores' ``blockwise_attention``) than decoded in registers per query.
+
+    The exact in-register kernel decodes every K/V vector again for each
+    query, so its time follows queries * tokens * q_heads: past 3e7
+    coordinates from 4 queries on, decoding once wins (D 128, 32 heads, 1,000
+    tokens: 84 -> 57 us at 8 queries; 4,096 tokens, 128 queries: 3,834 -> 71
+    us).  The score tables (``tables``) cost 15 to 27 us per query of 32 heads
+    whatever the window, decoding 3.3 us per 2^20 coordinates whatever the
+    queries: even near queries * q_heads * 2^18 = tokens * kv_heads * D (12,000
+    tokens x 32 heads: 120 against 150 us at 4 queries, 211 against 150 at 8).
+    The decoded window is at most 1 GiB for K and V together."""
+    if head_dim not in (64, 128) or kv_heads <= 0 or q_heads % kv_heads or q_heads // kv_heads not in (1, 2, 4, 8):
+        return False
+    window = tokens * kv_heads * head_dim
+    if queries < 4 or window > 1 << 28:
+        return False
+    if tables:
+        return queries * q_heads << 18 >= window
+    return queries * tokens * q_heads * head_dim >= 30_000_000
+
+
 def _ref_format_params(k_pq_cb: torch.Tensor, k_rvq_cb: Optional[torch.Tensor], rvq_subspaces: int,
                        sparse_k: int) -> "L.RefParams":
     M, Cn, d = k_pq_cb.shape

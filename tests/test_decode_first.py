@@ -1,0 +1,14 @@
+"""Which hybrid-attention calls decode their window once (kernels.decode_first)."""
+
+from apple_amd.kernels import decode_first
+
+
+def test_decode_first_lines():
+    assert not decode_first(1, 32, 32, 128, 24576, True)        # decode steps keep the score tables
+    assert not decode_first(3, 32, 32, 128, 100_000, False)     # and the in-register kernel
+    assert decode_first(128, 32, 32, 128, 4096, False)
+    assert decode_first(8, 32, 32, 128, 4096, True) and not decode_first(8, 32, 32, 128, 20_000, True)
+    assert not decode_first(64, 8, 8, 64, 64, False)            # launch-bound either way
+    assert not decode_first(128, 32, 32, 256, 4096, False)      # no matrix-core kernel of that head_dim
+    assert not decode_first(128, 24, 8, 128, 4096, False)       # nor of three query heads per KV head
+    assert not decode_first(128, 32, 32, 128, 70_000, False)    # a decoded window over 1 GiB

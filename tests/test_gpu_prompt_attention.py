@@ -73,3 +73,34 @@ def test_prompt_attention_strides_and_views(device):
     for qq in (q[1:].view(9, 3, 64), q[1:].view(9, 3, 64).clone()):
         got = K.blockwise_attention(qq, k, v, 0.125, False, None).double().cpu().numpy()
         assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + 5 * 2.0 ** -15)
+
+
+@pytest.mark.parametrize("fmt", ["gated", "subspace"])
+def test_hybrid_attention_decodes_once_for_many_queries(device, monkeypatch, fmt):
+    """A chunk past ``decode_first``'s line decodes both stores once and agrees with the decode-in-register
+    kernel (which a chunk below the line keeps) and with float64 over the decoded rows."""
+    import torch
+    from apple_amd import attention as A
+    from apple_amd import kernels as K
+    from apple_amd.quantization import HybridQuantizerMLX, _compress_tensor_sequence, _decode_compressed_tensor
+    from apple_amd.storage import RFSNConfig
+
+    B, Hq, Hkv, T, D = 150, 8, 4, 301, 128
+    ext = dict(rvq_subspaces=8, sparse_topk=4, rvq_codebook_size=256) if fmt == "subspace" else dict(rvq_codebook_size=64)
+    cfg = RFSNConfig(hidden_dim=Hq * D, num_heads=Hq, head_dim=D, num_kv_heads=Hkv, num_rvq_layers=3,
+                     rvq_sparsity_threshold=9.0, **ext)
+    g = torch.Generator().manual_seed(11)
+    qz = HybridQuantizerMLX(cfg, device=device, generator=g)
+    r = lambda *s: torch.randn(*s, generator=g).half().to(device)
+    ks, vs = (_compress_tensor_sequence(r(T, Hkv, D), qz) for _ in range(2))
+    q, pos = r(B, Hq, D), torch.arange(T - B, T, dtype=torch.int32, device=device)
+    assert K.decode_first(B, Hq, Hkv, D, T, False)
+    att = A.RFSNHybridAttentionMLX(cfg)
+    got = att(q, ks, vs, qz, causal=True, query_positions=pos)
+    monkeypatch.setattr(K, "decode_first", lambda *a: False)
+    reg = att(q, ks, vs, qz, causal=True, query_positions=pos)
+    k, v = (_decode_compressed_tensor(s, qz).cpu().numpy() for s in (ks, vs))
+    want = _ref(q.cpu().numpy(), k, v, D ** -0.5, np.repeat(pos.cpu().numpy()[:, None], Hq, 1))
+    for out in (got, reg):
+        err = np.abs(out.double().cpu().numpy() - want)
+        assert np.all(err <= np.abs(want) * 2.0 ** -11 + np.abs(v).max().astype(np.float64) * 2.0 ** -15)
