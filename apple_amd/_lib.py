@@ -80,6 +80,12 @@ class RefParams(C.Structure):
                 ("score_tables", i32), ("table_tol", f32), ("table_stats", vp), ("drift", vp)]
 
 
+class LinearParams(C.Structure):
+    _fields_ = [("x", vp), ("rows", i64), ("k", i32), ("mode", i32), ("w", vp * 3), ("out", vp * 3), ("n", i32 * 3),
+                ("norm_eps", f32), ("norm_w", vp), ("xn", vp), ("residual", vp), ("head_dim", i32), ("pos0", i64),
+                ("inv_freq", vp), ("cos", vp), ("sin", vp)]
+
+
 class EncodeJob(C.Structure):
     _fields_ = [("x", vp), ("n", i64), ("ldx", i64), ("pq_cb", vp), ("rvq_cb", vp), ("out", Codes)]
 
@@ -113,6 +119,7 @@ SIGNATURES = {
     "rfsn_decode_ref": (i32, [vp, i64, i32, i32, i32, vp, vp, vp, i64, i32, i32, vp, vp, vp]),
     "rfsn_attention_workspace_bytes": (sz, [i32, i32, i32, i32]),
     "rfsn_blockwise_attention": (i32, [vp, i32, i32, i32, vp, vp, i64, i32, i64, i64, f32, i32, vp, vp, vp, sz, vp]),
+    "rfsn_layer_linear": (i32, [C.POINTER(LinearParams), vp]),
     "rfsn_pack_codes": (i32, [vp, i64, i64, i32, i32, vp, i64, i64, vp]),
     "rfsn_pack_score_codes": (i32, [vp, vp, vp, vp, i32, i64, i32, vp, vp, vp, vp, i64, i64, vp]),
     "rfsn_warm_append_pair": (i32, [C.POINTER(Format), C.POINTER(Codes), C.POINTER(Codes), i64, i32, vp, vp, vp,

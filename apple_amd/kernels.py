@@ -690,6 +690,59 @@ def fused_attention(q: torch.Tensor, fmt: WarmFormat, *, kv_heads: int, scale: f
 
 
 # --------------------------------------------------------------------------
+# decoder layer projections (llama32_adapter.py:555-587)
+# --------------------------------------------------------------------------
+
+LINEAR_PLAIN, LINEAR_SWIGLU, LINEAR_RESIDUAL = 0, 1, 2
+
+
+def layer_linear_ok(k: int, sizes: Sequence[int], head_dim: int = 0) -> bool:
+    """Whether ``rfsn_layer_linear`` serves projections of ``k`` inputs to ``sizes`` outputs."""
+    unit = head_dim if head_dim else 4
+    return (64 <= k <= 32768 and k % 64 == 0 and all(n > 0 and n % unit == 0 and n % 4 == 0 for n in sizes)
+            and sum(sizes) < 1 << 28 and head_dim % 8 == 0)
+
+
+def layer_linear(x: torch.Tensor, weights: Sequence[torch.Tensor], mode: int = LINEAR_PLAIN, *,
+                 norm: Optional[Tuple[torch.Tensor, float]] = None, residual: Optional[torch.Tensor] = None,
+                 head_dim: int = 0, tables: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+                 inv_freq: Optional[torch.Tensor] = None, pos0: int = 0) -> List[torch.Tensor]:
+    """Projections of x [rows, k] fp16 by fp32 ``weights`` [n, k] (one launch
+    for one row), each result fp16 [rows, n] (``rfsn_layer_linear``).
+
+    ``norm`` = (weight fp32 [k], eps): RMSNorm of x first.  LINEAR_PLAIN with
+    ``head_dim``: rotary embedding on the first two outputs, the angles from
+    ``inv_freq`` (float64 [head_dim / 2], row s at position pos0 + s) or
+    ``tables`` (cos, sin fp32 [rows, head_dim]).  LINEAR_SWIGLU: (gate, up) ->
+    [act * up].  LINEAR_RESIDUAL: [residual + x W^T]."""
+    rows, k = x.shape
+    outs = [torch.empty((rows, w.shape[0]), dtype=torch.float16, device=x.device)
+            for w in (weights[:1] if mode == LINEAR_SWIGLU else weights)]
+    p = L.LinearParams()
+    p.x, p.rows, p.k, p.mode = x.data_ptr(), rows, k, mode
+    for i, w in enumerate(weights):
+        p.w[i], p.n[i] = w.data_ptr(), w.shape[0]
+    for i, o in enumerate(outs):
+        p.out[i] = o.data_ptr()
+    xn = None
+    if norm is not None:
+        p.norm_w, p.norm_eps = norm[0].data_ptr(), norm[1]
+        if rows > 1:
+            xn = torch.empty_like(x)
+            p.xn = xn.data_ptr()
+    if residual is not None:
+        p.residual = residual.data_ptr()
+    if head_dim:
+        p.head_dim, p.pos0 = head_dim, pos0
+        if inv_freq is not None:
+            p.inv_freq = inv_freq.data_ptr()
+        else:
+            p.cos, p.sin = tables[0].data_ptr(), tables[1].data_ptr()
+    L.call("rfsn_layer_linear", C.byref(p), _stream(x))
+    return outs
+
+
+# --------------------------------------------------------------------------
 # reference-format attention (PQ + gated full-dimension RVQ, decoded on the fly)
 # --------------------------------------------------------------------------
 

@@ -10,11 +10,16 @@ decode path.
   are (``num_kv_heads``); the reference repeats them to the query heads
   first (llama32_adapter.py:380-386, 578-579).
 
-Norms, projections, activations and the dense prompt attention are torch
-ops on the GPU, computed in fp32 from fp16 activations with fp16 results at
-the reference's cast points.  Cache-backed decode goes through the cache's
-fused dequant-attention kernel.  Weights are module parameters: the
-reference's initialisation or a local state dict; nothing is downloaded.
+Norms, projections and activations are computed in fp32 from fp16
+activations with fp16 results at the reference's cast points: by torch ops
+in the reference's layer, and in the Llama layer by ``rfsn_layer_linear``
+(RMSNorm, projection, rotary embedding / SwiGLU / residual in one pass over
+the weights) with the prompt's attention on the matrix cores; where autograd,
+a tracer, autocast or a tensor subclass watches the call, or weights are not
+plain fp32 matrices, the Llama layer runs the same steps as torch ops.
+Cache-backed decode goes through the cache's fused dequant-attention kernel.
+Weights are module parameters: the reference's initialisation or a local
+state dict; nothing is downloaded.
 """
 
 from __future__ import annotations
@@ -27,6 +32,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from . import kernels as K
 from .cache import RFSNv10KVCacheMLX
 from .quantization import HybridQuantizerMLX
 from .storage import AsyncHierarchicalRouterMLX, RFSNConfig
@@ -82,6 +88,23 @@ def _rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float) -> to
     if weight is not None:
         y = y * weight.float()
     return y.to(torch.float16)
+
+
+def _unwatched(x: torch.Tensor) -> bool:
+    """Whether a call on ``x`` may pass torch's operators by: nothing records
+    gradients of it (reverse or forward mode), maps, traces or compiles it,
+    intercepts its operators or casts them, and it is a plain tensor."""
+    return (type(x) is torch.Tensor and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
+            and torch._C._get_tracing_state() is None and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0 and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x))
+
+
+def _plain_weight(w: torch.Tensor, device: torch.device) -> bool:
+    """A weight the projection kernel reads as it is: fp32, contiguous, aligned, on the device, not trained."""
+    return (w.dtype is torch.float32 and w.device == device and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and not (w.requires_grad and torch.is_grad_enabled()) and type(w) in (torch.nn.Parameter, torch.Tensor))
 
 
 class RFSNDecoderLayerMLX(torch.nn.Module):
@@ -168,9 +191,10 @@ class RFSNDecoderLayerMLX(torch.nn.Module):
             window = context_window
             if window is None:
                 window = max(self.config.block_size_seq, min(self.cache.total_tokens, self.config.warm_capacity))
+            # the query is the newest token: attention_forward's default position
+            # (a device tensor here would be read back to the host for the window)
             attended = self.cache.attention_forward(
-                q[:, 0], causal=True, query_positions=torch.tensor([pos], dtype=torch.int32, device=self.device),
-                router=router, current_position=pos, context_window=window,
+                q[:, 0], causal=True, router=router, current_position=pos, context_window=window,
             ).reshape(1, 1, self.num_heads, self.head_dim)
         else:
             rep = self.num_heads // self.num_kv_heads
@@ -276,6 +300,7 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         shapes = {"input_layernorm": (D,), "post_attention_layernorm": (D,), "q_proj": (H * self.head_dim, D),
                   "k_proj": (Hkv * self.head_dim, D), "v_proj": (Hkv * self.head_dim, D),
                   "o_proj": (D, H * self.head_dim), "gate_proj": (I, D), "up_proj": (I, D), "down_proj": (D, I)}
+        self._shapes = {n: torch.Size(s) for n, s in shapes.items()}
         g = generator if generator is not None else torch.Generator().manual_seed(4321 + layer_idx)
         for name in self.WEIGHTS:
             if weights is not None:
@@ -325,6 +350,50 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
                          for t in (cos, sin))
         return rope_cos_sin(pid, self.head_dim, self.rope_theta, self.rope_scaling)
 
+    def _native(self, h16: torch.Tensor) -> bool:
+        """Whether ``rfsn_layer_linear`` runs this call's projections: a plain
+        [1, S, hidden] fp16 input nothing watches, weights as it reads them."""
+        D, qkv = self.hidden_dim, (self.num_heads + 2 * self.num_kv_heads) * self.head_dim
+        if (not _unwatched(h16) or h16.dim() != 3 or h16.shape[1] == 0 or int(h16.shape[2]) != D or not h16.is_cuda
+                or h16.device.index != torch.cuda.current_device()):
+            return False
+        for name, shape in self._shapes.items():
+            w = self._parameters.get(name)
+            if w is None or w.shape != shape or not _plain_weight(w, h16.device):
+                return False
+        inter = self._shapes["gate_proj"][0]
+        return (K.layer_linear_ok(D, (qkv, ), self.head_dim) and K.layer_linear_ok(D, (inter, inter))
+                and K.layer_linear_ok(self.num_heads * self.head_dim, (D,)) and K.layer_linear_ok(inter, (D,)))
+
+    def _rows(self, h16: torch.Tensor) -> torch.Tensor:
+        """[1, S, hidden] as the contiguous, aligned rows [S, hidden] the projection kernel reads."""
+        x = h16.reshape(-1, self.hidden_dim).contiguous()
+        return x.clone() if x.data_ptr() % 16 else x
+
+    def _inv_freq(self) -> torch.Tensor:
+        """``rope_inv_freq`` on the device, rebuilt when the layer's rotary settings change."""
+        key = (self.head_dim, self.rope_theta, None if not self.rope_scaling else dict(self.rope_scaling))
+        if getattr(self, "_inv_freq_key", None) != key:
+            self._inv_freq_memo = rope_inv_freq(*key, self.device).contiguous()
+            self._inv_freq_key = key
+        return self._inv_freq_memo
+
+    def _qkv(self, h16: torch.Tensor, native: bool, position_embeddings, position_ids):
+        """Rotated q and k, and v, [1, S, heads, head_dim] (llama32_adapter.py:570-580)."""
+        S = int(h16.shape[1])
+        if not native:
+            return self._project_qkv(h16, *self._positions(S, position_embeddings, position_ids))
+        w = self._parameters
+        if position_embeddings is None and position_ids is None and self.rotary_module is None:
+            rope = dict(inv_freq=self._inv_freq(), pos0=self.cache.total_tokens)
+        else:
+            cos, sin = self._positions(S, position_embeddings, position_ids)
+            shape = (S, self.head_dim)
+            rope = dict(tables=(cos.expand(shape).contiguous(), sin.expand(shape).contiguous()))
+        outs = K.layer_linear(self._rows(h16), [w["q_proj"], w["k_proj"], w["v_proj"]], head_dim=self.head_dim,
+                              norm=(w["input_layernorm"], self.rms_norm_eps), **rope)
+        return tuple(o.view(1, S, -1, self.head_dim) for o in outs)
+
     def _project_qkv(self, h16: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
         """llama32_adapter.py:570-580 without the KV repeat (the cache groups heads)."""
         n = _rms_norm(h16, self.input_layernorm, self.rms_norm_eps)
@@ -356,8 +425,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         S = int(hidden_states.shape[1])
         if S == 0:
             return
-        cos, sin = self._positions(S, position_embeddings, position_ids)
-        _, k, v = self._project_qkv(hidden_states.to(self.device, torch.float16), cos, sin)
+        h16 = hidden_states.to(self.device, torch.float16)
+        _, k, v = self._qkv(h16, self._native(h16), position_embeddings, position_ids)
         self.cache.update(k[0], v[0], self.quantizer, disk_dir=self.disk_cache_dir)
 
     def forward(self, hidden_states: torch.Tensor, position_embeddings=None, position_ids=None,
@@ -367,21 +436,32 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         if int(hidden_states.shape[0]) != 1:
             raise ValueError("The Llama adapter currently supports batch size 1 only")
         S = int(hidden_states.shape[1])
-        cos, sin = self._positions(S, position_embeddings, position_ids)
         residual = hidden_states.to(self.device, torch.float16)
-        q, k, v = self._project_qkv(residual, cos, sin)
+        native = self._native(residual)
+        q, k, v = self._qkv(residual, native, position_embeddings, position_ids)
         if use_cache:
             if S != 1:
                 raise ValueError("cache-backed decode expects input shape [1, 1, hidden_dim]")
             self.cache.update(k[0], v[0], self.quantizer, disk_dir=self.disk_cache_dir)
             pos = self.cache.total_tokens - 1
             attended = self.cache.attention_forward(
-                q[:, 0], causal=True, query_positions=torch.tensor([pos], dtype=torch.int32, device=self.device),
-                router=router, current_position=pos, context_window=context_window,
+                q[:, 0], causal=True, router=router, current_position=pos, context_window=context_window,
             ).reshape(1, 1, self.num_heads, self.head_dim)
+        elif native and S and self.head_dim in (64, 128) and self.num_key_value_groups in (1, 2, 4, 8):
+            own = torch.arange(S, dtype=torch.int32, device=self.device)[:, None].expand(S, self.num_heads)
+            attended = K.blockwise_attention(q[0], k[0], v[0], self.scale, True, own)
         else:
             g = self.num_key_value_groups
             attended = _dense_exact_attention(q, _repeat_kv(k, g), _repeat_kv(v, g), self.scale, causal=True)
-        attn = _project(attended.reshape(1, S, self.num_heads * self.head_dim), self.o_proj)
+        attended = attended.reshape(1, S, self.num_heads * self.head_dim)
+        if native:
+            w = self._parameters
+            hidden, = K.layer_linear(attended.reshape(S, -1), [w["o_proj"]], K.LINEAR_RESIDUAL,
+                                     residual=self._rows(residual))
+            act, = K.layer_linear(hidden, [w["gate_proj"], w["up_proj"]], K.LINEAR_SWIGLU,
+                                  norm=(w["post_attention_layernorm"], self.rms_norm_eps))
+            out, = K.layer_linear(act, [w["down_proj"]], K.LINEAR_RESIDUAL, residual=hidden)
+            return out.reshape(1, S, self.hidden_dim)
+        attn = _project(attended, self.o_proj)
         hidden = residual + attn
         return hidden + self._mlp(hidden)

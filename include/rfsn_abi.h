@@ -201,6 +201,44 @@ int rfsn_blockwise_attention(const void* q_dev, int32_t B, int32_t Hq, int32_t D
                              const int32_t* qpos_dev, void* out_dev,
                              void* workspace_dev, size_t workspace_bytes, void* stream);
 
+/* ---------------------------------------------------------------- decoder layer
+ * y = x W^T of the decoder layer's projections (llama32_adapter.py:555-587):
+ * x [rows][k] fp16 (contiguous), up to three weight matrices W_t [n_t][k]
+ * fp32 with outputs out_t [rows][n_t] fp16.
+ *  - norm_w (or NULL): x is RMS-normed first, fp16(x * rsqrt(mean(x^2) + eps)
+ *    * norm_w); xn = scratch for the normed rows, fp16 [rows][k], needed when
+ *    rows > 1.
+ *  - mode 0: out_t = fp16(x W_t^T); with head_dim > 0, rotary embedding on
+ *    out_0 and out_1 (heads of head_dim): fp16(v cos + rotate_half(v) sin) of
+ *    the rounded values, the angles of row s from inv_freq (float64
+ *    [head_dim / 2], position pos0 + s) or, when NULL, from cos / sin fp32
+ *    [rows][head_dim].
+ *  - mode 1 (SwiGLU, n_0 == n_1): out_0 = fp16(act * up), up = fp16(x W_1^T),
+ *    act = fp16(g * sigmoid(g)), g = fp16(x W_0^T).
+ *  - mode 2: out_0 = fp16(residual + fp16(x W_0^T)), residual [rows][n_0].
+ * Sums are fp32; weights keep their fp32 value to 23 bits or 2^-37.
+ * k a multiple of 64 up to 32768, n_t multiples of 4 (of head_dim with rotary
+ * embedding), buffers 16-byte aligned. */
+typedef struct rfsn_linear_params {
+  const void* x;
+  int64_t rows;
+  int32_t k;
+  int32_t mode;
+  const float* w[3];
+  void* out[3];
+  int32_t n[3];
+  float norm_eps;
+  const float* norm_w;
+  void* xn;
+  const void* residual;
+  int32_t head_dim;
+  int64_t pos0;
+  const double* inv_freq;
+  const float* cos;
+  const float* sin;
+} rfsn_linear_params;
+int rfsn_layer_linear(const rfsn_linear_params* p, void* stream);
+
 /* Code layout the fused kernel streams ("tiled"): codes of one KV head live
  * in a block of cap*M bytes (cap a multiple of 32); inside 32-token tile
  * tau, the code of (token t, subspace m) sits at byte
