@@ -701,7 +701,7 @@ sparse_topk64_kernel(const uint16_t* __restrict__ x, int64_t n, int64_t ldx, con
 // ---------------------------------------------------------------- fused warm encode
 // One launch encodes up to kMaxJobs vector sets (a chunk's K and V): PQ, the
 // subspace RVQ stage on the register-resident fp16 PQ residual, then the
-// top-k |r2|, head_dim 64.  A block (16 waves) holds 256 vectors of one job
+// top-k |r2|, head_dim 64.  A block of W waves holds 16 W vectors of one job
 // and first writes the augmented centroid rows of every (stage, subspace)
 // into LDS: coordinates in 8-byte groups, then (R/2 hi, R/2 lo, 1, 1), with
 // R the canonical fl32(S c*c); rows past the codebook get R/2 = +inf.  A wave
@@ -715,9 +715,6 @@ sparse_topk64_kernel(const uint16_t* __restrict__ x, int64_t n, int64_t ldx, con
 // never leaves registers; each lane folds its share of the vector's r2 into a
 // running top-k, and the codes are written once per vector at the end.
 constexpr int kMaxJobs = 4;
-constexpr int kFeWaves = 16;
-constexpr int kFeThreads = kFeWaves * 64;
-constexpr int kFeVecs = kFeWaves * 16;  // vectors per block
 
 struct EncodeJob {
   const uint16_t* x;
@@ -770,8 +767,9 @@ __device__ __forceinline__ void key_insert3(int& m1, int& m2, int& m3, int k) {
 __device__ __forceinline__ int lane_xor16(int v) { return __builtin_amdgcn_ds_swizzle(v, 0x401F); }
 __device__ __forceinline__ int lane_xor32(int v, int xor32_addr) { return __builtin_amdgcn_ds_bpermute(xor32_addr, v); }
 
-template <int DS, bool RVQ, int KS>
-__global__ void __launch_bounds__(kFeThreads, 1) warm_encode_fused_kernel(const EncodeJobs jobs) {
+template <int DS, bool RVQ, int KS, int W>
+__global__ void __launch_bounds__(W * 64, 1) warm_encode_fused_kernel(const EncodeJobs jobs) {
+  constexpr int kFeThreads = W * 64, kFeVecs = W * 16;
   constexpr int M = 64 / DS;
   constexpr int S = RVQ ? 2 : 1;       // stages
   constexpr int CG = DS / 4;           // coordinate k-groups of a row
@@ -979,47 +977,74 @@ __global__ void __launch_bounds__(kFeThreads, 1) warm_encode_fused_kernel(const 
       key_insert3(p1, p2, p3, o2);
       key_insert3(p1, p2, p3, o3);
     }
-    if (unique) return m1 & 0xFF;
-    double xs[DS];
-    double lacc = 0.0;
-#pragma unroll
-    for (int k = 0; k < DS / 2; ++k) {
-      const h2 x2 = pair(xw[k]);
-      xs[2 * k] = (double)(float)x2[0];
-      xs[2 * k + 1] = (double)(float)x2[1];
-      lacc = __builtin_fma(xs[2 * k], xs[2 * k], lacc);
-      lacc = __builtin_fma(xs[2 * k + 1], xs[2 * k + 1], lacc);
-    }
-    const float L = (float)lacc;
     const float w1 = key_value(p1), w3 = key_value(p3);
     const bool pair3 = safe && w3 - w1 > 2.0f * E + 0x1p-14f * (fabsf(w1) + fabsf(w3));
+    // a vector's canonical terms: its coordinates and fl32(L) as a float64 chain
+    struct Exact {
+      double xs[DS];
+      float L;
+    };
+    auto terms = [&](const uint32_t (&w)[DS / 2]) {
+      Exact e;
+      double lacc = 0.0;
+#pragma unroll
+      for (int k = 0; k < DS / 2; ++k) {
+        const h2 x2 = pair(w[k]);
+        e.xs[2 * k] = (double)(float)x2[0];
+        e.xs[2 * k + 1] = (double)(float)x2[1];
+        lacc = __builtin_fma(e.xs[2 * k], e.xs[2 * k], lacc);
+        lacc = __builtin_fma(e.xs[2 * k + 1], e.xs[2 * k + 1], lacc);
+      }
+      e.L = (float)lacc;
+      return e;
+    };
     // canonical distance of centroid j: fl32(fl32(L - 2X) + R), X and R float64 chains
-    auto exact = [&](int j) {
+    auto exact = [&](const Exact& e, int j) {
       const uint8_t* row = tb + j * RB;
       double xa = 0.0, ra = 0.0;
 #pragma unroll
       for (int u = 0; u < DS; ++u) {
         const double c = (double)h2f(reinterpret_cast<const uint16_t*>(row)[u]);
-        xa = __builtin_fma(xs[u], c, xa);
+        xa = __builtin_fma(e.xs[u], c, xa);
         ra = __builtin_fma(c, c, ra);
       }
-      return __fadd_rn(__fsub_rn(L, 2.0f * (float)xa), (float)ra);
+      return __fadd_rn(__fsub_rn(e.L, 2.0f * (float)xa), (float)ra);
     };
-    int code;
-    if (pair3) {
+    int code = m1 & 0xFF;
+    if (!unique && pair3) {
+      const Exact e = terms(xw);
       const int ja = min(p1 & 0xFF, p2 & 0xFF), jb = max(p1 & 0xFF, p2 & 0xFF);
-      const float da = exact(ja), db = exact(jb);
+      const float da = exact(e, ja), db = exact(e, jb);
       code = db < da ? jb : ja;  // first min: ties keep the lower index
-    } else {
+    }
+    // Vectors that more than two centroids may claim: the whole codebook, one vector
+    // at a time with its centroids spread over the wave's lanes (a lane alone takes
+    // 16 us over 256 of them, which one such vector in a launch used to add to it).
+    for (uint64_t rest = __builtin_amdgcn_ballot_w64(!unique && !pair3) & 0xFFFF; rest != 0; rest &= rest - 1) {
+      const int src = __builtin_ctzll(rest);  // lanes src, src + 16, ... hold the vector
+      uint32_t w[DS / 2];
+#pragma unroll
+      for (int k = 0; k < DS / 2; ++k) w[k] = (uint32_t)__builtin_amdgcn_readlane((int)xw[k], src);
+      const Exact e = terms(w);
       float best = __builtin_inff();
-      code = 0;
-      for (int j = 0; j < nc; ++j) {
-        const float dj = exact(j);
+      int bj = 256;
+      for (int j = lane; j < nc; j += 64) {
+        const float dj = exact(e, j);
         if (dj < best) {
           best = dj;
-          code = j;
+          bj = j;
         }
       }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const float ob = __shfl_xor(best, o, 64);
+        const int oj = __shfl_xor(bj, o, 64);
+        if (ob < best || (ob == best && oj < bj)) {
+          best = ob;
+          bj = oj;
+        }
+      }
+      if (vi == src) code = bj < 256 ? bj : 0;  // nothing below +inf: the first
     }
     return code;
   };
@@ -1668,10 +1693,24 @@ bool fused_encode_ok(const rfsn_format* f, const EncodeJob& j) {
 }
 
 int launch_warm_encode_fused(const rfsn_format* f, EncodeJobs& jobs, hipStream_t s) {
-  int blocks = 0;
+  // Waves per block.  A block's tables take most of a CU's LDS, so blocks run 256 at
+  // a time, and such a round costs about 15 + 1.75 W us (4, 8, 16 waves: 22, 28, 43
+  // us at M 8 + RVQ 8 + top-4): the W whose rounds cost least.  32,768 vectors: 28
+  // us in 256 blocks of 8 waves, 43 in 128 of 16.
+  int W = 16, blocks = 0;
+  int64_t least = INT64_MAX;
+  for (int w = 16; w >= 4; w /= 2) {
+    int64_t b = 0;
+    for (int i = 0; i < jobs.count; ++i) b += ceil_div(jobs.j[i].n, 16 * w);
+    const int64_t cost = ceil_div(b, 256) * (60 + 7 * w);
+    if (cost < least) {
+      least = cost;
+      W = w;
+    }
+  }
   for (int i = 0; i < jobs.count; ++i) {
     jobs.j[i].block0 = blocks;
-    blocks += (int)ceil_div(jobs.j[i].n, kFeVecs);
+    blocks += (int)ceil_div(jobs.j[i].n, 16 * W);
   }
   if (blocks == 0) return RFSN_OK;
   jobs.C = f->pq_centroids;
@@ -1679,7 +1718,14 @@ int launch_warm_encode_fused(const rfsn_format* f, EncodeJobs& jobs, hipStream_t
   const int d = f->head_dim / f->pq_subspaces;
   const bool rvq = f->rvq_subspaces > 0;
   const bool ks = f->sparse_k > 0;
-#define RFSN_FE(DS, R, K) hipLaunchKernelGGL((warm_encode_fused_kernel<DS, R, K>), dim3(blocks), dim3(kFeThreads), 0, s, jobs)
+#define RFSN_FE_W(DS, R, K, WW) \
+  hipLaunchKernelGGL((warm_encode_fused_kernel<DS, R, K, WW>), dim3(blocks), dim3(WW * 64), 0, s, jobs)
+#define RFSN_FE(DS, R, K)                   \
+  do {                                      \
+    if (W == 16) RFSN_FE_W(DS, R, K, 16);   \
+    else if (W == 8) RFSN_FE_W(DS, R, K, 8); \
+    else RFSN_FE_W(DS, R, K, 4);            \
+  } while (0)
   if (d == 8) {
     if (rvq) { if (ks) RFSN_FE(8, true, 4); else RFSN_FE(8, true, 0); }
     else { if (ks) RFSN_FE(8, false, 4); else RFSN_FE(8, false, 0); }
@@ -1687,6 +1733,7 @@ int launch_warm_encode_fused(const rfsn_format* f, EncodeJobs& jobs, hipStream_t
     if (rvq) { if (ks) RFSN_FE(4, true, 4); else RFSN_FE(4, true, 0); }
     else { if (ks) RFSN_FE(4, false, 4); else RFSN_FE(4, false, 0); }
   }
+#undef RFSN_FE_W
 #undef RFSN_FE
   return check_launch("warm_encode_fused");
 }
