@@ -192,8 +192,8 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def stream_handle(device: Optional[torch.device] = None) -> int:
     """The current torch stream of ``device`` as a hipStream_t."""
-    if isinstance(device, torch.device) and device.index is not None:
-        return torch._C._cuda_getCurrentRawStream(device.index)  # no Stream object built
+    if isinstance(device, torch.device):  # no Stream object built
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -560,6 +560,17 @@ class RFSNv10KVCacheMLX:
             "cold_chunk_cache_misses": 0,
         }
 
+    def whole_window_stats(self) -> Dict[str, int]:
+        """The access counters of one query token over the hot and warm tiers
+        (no cold tier), as ``attention_forward`` leaves them (cache.py:250-342)."""
+        stats = self._empty_access_stats()
+        stats["window_end"] = stats["window_tokens"] = self.total_tokens
+        stats["hot_tokens_materialized"] = self.num_hot
+        stats["warm_tokens_materialized"] = stats["reconstructed_tokens"] = self.num_warm
+        stats["warm_chunk_decodes"] = self._warm_chunks((0, self.num_warm)) if self.num_warm else 0
+        stats["query_tokens"] = 1
+        return stats
+
     def get_last_access_stats(self) -> Dict[str, int]:
         return dict(self.last_access_stats)
 
@@ -1834,6 +1845,7 @@ class DecodeSession:
         self._layout: Optional[tuple] = None  # the cache's segment layout at the last rebuild
         self._rows: Optional[tuple] = None  # the last fast step's new rows (read by its launch)
         self.rebuilds = 0
+        self.left: Optional[tuple] = None  # ``state`` after the last step, for a holder that compares it
         self.regrows = 0  # steps whose update kept the segments in place (launch patched, not rebuilt)
 
     def _chunk_set(self, total: Optional[int] = None) -> Optional[List[int]]:
@@ -1890,6 +1902,29 @@ class DecodeSession:
             return self.out
         self._rebuild(ids)
         return self.out
+
+    def state(self) -> tuple:
+        """What the prepared launch was built from, beyond what ``step`` itself
+        tracks: a holder that shares the cache with other writers drops the
+        launch (``forget``) when this differs from its value after the last
+        step."""
+        c = self.cache
+        return (c.total_tokens, c.num_hot, c._hot_head, c.num_warm, c.num_cold, c._hot_k.data_ptr(),
+                c.config.score_table_tolerance, c.config.fused_score_tables,
+                None if c._kq is None else c._codebook_key(bool(c._fmt().rvq_subspaces)))
+
+    def forget(self) -> None:
+        """Drop the prepared launch: the next step builds it anew."""
+        self._launch, self._ids = None, None
+
+    def splits_stale(self) -> bool:
+        """Whether the window has grown enough since the last rebuild for the
+        automatic split count to have moved by more than an eighth."""
+        p = None if self._launch is None else self._launch.params
+        if p is None:
+            return False
+        now = K.fused_splits(p.batch, p.q_heads, p.kv_heads, p.hot_len, p.max_tokens, p.max_segments)
+        return 8 * abs(now - p.splits) > p.splits
 
     def _rebuild(self, ids: Optional[List[int]]) -> None:
         c = self.cache

@@ -706,7 +706,8 @@ def layer_linear_ok(k: int, sizes: Sequence[int], head_dim: int = 0) -> bool:
 def layer_linear(x: torch.Tensor, weights: Sequence[torch.Tensor], mode: int = LINEAR_PLAIN, *,
                  norm: Optional[Tuple[torch.Tensor, float]] = None, residual: Optional[torch.Tensor] = None,
                  head_dim: int = 0, tables: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-                 inv_freq: Optional[torch.Tensor] = None, pos0: int = 0) -> List[torch.Tensor]:
+                 inv_freq: Optional[torch.Tensor] = None, pos0: int = 0,
+                 out0: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
     """Projections of x [rows, k] fp16 by fp32 ``weights`` [n, k] (one launch
     for one row), each result fp16 [rows, n] (``rfsn_layer_linear``).
 
@@ -714,10 +715,11 @@ def layer_linear(x: torch.Tensor, weights: Sequence[torch.Tensor], mode: int = L
     ``head_dim``: rotary embedding on the first two outputs, the angles from
     ``inv_freq`` (float64 [head_dim / 2], row s at position pos0 + s) or
     ``tables`` (cos, sin fp32 [rows, head_dim]).  LINEAR_SWIGLU: (gate, up) ->
-    [act * up].  LINEAR_RESIDUAL: [residual + x W^T]."""
+    [act * up].  LINEAR_RESIDUAL: [residual + x W^T].  ``out0``: the buffer of
+    the first result (contiguous fp16 [rows, n_0]) instead of a new one."""
     rows, k = x.shape
-    outs = [torch.empty((rows, w.shape[0]), dtype=torch.float16, device=x.device)
-            for w in (weights[:1] if mode == LINEAR_SWIGLU else weights)]
+    outs = [torch.empty((rows, w.shape[0]), dtype=torch.float16, device=x.device) if i or out0 is None else out0
+            for i, w in enumerate(weights[:1] if mode == LINEAR_SWIGLU else weights)]
     p = L.LinearParams()
     p.x, p.rows, p.k, p.mode = x.data_ptr(), rows, k, mode
     for i, w in enumerate(weights):

@@ -378,7 +378,38 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
             self._inv_freq_key = key
         return self._inv_freq_memo
 
-    def _qkv(self, h16: torch.Tensor, native: bool, position_embeddings, position_ids):
+    def _session(self):
+        """The decode session of a cached step over the whole hot + warm window
+        (``DecodeSession``: most steps re-issue one prepared launch, which
+        appends the token itself), or None where the general ``update`` +
+        ``attention_forward`` has to run: a cold tier, or a step that may spill
+        into one, another tier policy, or a format the fused kernel does not
+        serve.  A cache that was written, reconfigured or recalibrated since
+        the session's last step has its launch built anew."""
+        c = self.cache
+        if (not c._recency or not c._subspace or c.num_cold or c._kq is None or c.hot_capacity < 2 * c.HOT_BLOCK
+                or c.num_warm + c.HOT_BLOCK > c.warm_capacity or not c._fused_ok(self.num_heads)):
+            return None
+        s = getattr(self, "_decode", None)
+        if s is None or s.cache is not c or s.quantizer is not self.quantizer:
+            q = torch.empty((1, self.num_heads, self.head_dim), dtype=torch.float16, device=c._hot_k.device)
+            s = self._decode = c.decode_session(q, self.quantizer)
+        elif s.left != s.state() or s.splits_stale():
+            s.forget()
+        return s
+
+    def __getstate__(self):
+        # the session's prepared launch holds device addresses: a copy of the layer builds its own
+        return {n: v for n, v in self.__dict__.items() if n != "_decode"}
+
+    def _session_step(self, session, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+        session.left = None  # a step that raises leaves a launch to rebuild
+        out = session.step(k, v)
+        self.cache.last_access_stats = self.cache.whole_window_stats()
+        session.left = session.state()
+        return out
+
+    def _qkv(self, h16: torch.Tensor, native: bool, position_embeddings, position_ids, q_out=None):
         """Rotated q and k, and v, [1, S, heads, head_dim] (llama32_adapter.py:570-580)."""
         S = int(h16.shape[1])
         if not native:
@@ -391,7 +422,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
             shape = (S, self.head_dim)
             rope = dict(tables=(cos.expand(shape).contiguous(), sin.expand(shape).contiguous()))
         outs = K.layer_linear(self._rows(h16), [w["q_proj"], w["k_proj"], w["v_proj"]], head_dim=self.head_dim,
-                              norm=(w["input_layernorm"], self.rms_norm_eps), **rope)
+                              norm=(w["input_layernorm"], self.rms_norm_eps),
+                              out0=None if q_out is None else q_out.view(1, -1), **rope)
         return tuple(o.view(1, S, -1, self.head_dim) for o in outs)
 
     def _project_qkv(self, h16: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
@@ -438,8 +470,14 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         S = int(hidden_states.shape[1])
         residual = hidden_states.to(self.device, torch.float16)
         native = self._native(residual)
-        q, k, v = self._qkv(residual, native, position_embeddings, position_ids)
-        if use_cache:
+        session = None
+        if use_cache and native and S == 1 and router is None and context_window is None:
+            session = self._session()
+        q, k, v = self._qkv(residual, native, position_embeddings, position_ids,
+                            None if session is None else session.q)
+        if session is not None:
+            attended = self._session_step(session, k[0], v[0])
+        elif use_cache:
             if S != 1:
                 raise ValueError("cache-backed decode expects input shape [1, 1, hidden_dim]")
             self.cache.update(k[0], v[0], self.quantizer, disk_dir=self.disk_cache_dir)

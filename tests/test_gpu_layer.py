@@ -201,3 +201,50 @@ def test_llama_layer_cpu_rotary_module(device, tmp_path):
         outs.append(H(layer(x, use_cache=True)))
     assert rot.calls >= 2
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+def test_llama_layer_session_follows_its_cache(device, tmp_path):
+    """The layer's cached steps through its decode session against the general update + attention_forward: the
+    same cache rows and access counters and attention within a rounding of fp16, over demotions, writes and
+    recalibration from outside between steps, another stream, a smaller window, the first cold spill and a reset."""
+    from apple_amd.layer import Llama32DecoderLayerMLX
+
+    layers = []
+    for sub in ("a", "b"):
+        cfg = _ext_config(tmp_path / sub, warm_capacity=192)
+        layers.append(Llama32DecoderLayerMLX(cfg, intermediate_size=256, device=device,
+                                             quantizer=_ext_quantizer(cfg, device, 8),
+                                             generator=torch.Generator().manual_seed(4)))
+    ours, general = layers
+    general._session = lambda: None
+    g = rng(35)
+    t = lambda *s: torch.from_numpy(randn16(g, *s)).to(device)
+    prompt = t(1, 90, 512)
+    for layer in layers:
+        layer.prefill_cache(prompt)
+    used = 0
+    for step in range(150):
+        if step in (7, 40):                      # tokens written past the layer
+            k, v = t(step, 4, 64), t(step, 4, 64)
+            for layer in layers:
+                layer.cache.update(k, v, layer.quantizer)
+        if step == 20:                           # codebooks recalibrated in place
+            for layer in layers:
+                layer.quantizer.pq.codebooks.mul_(1.01)
+        kw = dict(context_window=70) if step in (11, 12) else {}
+        x = t(1, 1, 512)
+        with torch.cuda.stream(torch.cuda.Stream(device) if step in (30, 31) else torch.cuda.current_stream(device)):
+            torch.cuda.synchronize()
+            outs = [layer(x, use_cache=True, **kw) for layer in layers]
+            torch.cuda.synchronize()
+        used += ours._session() is not None
+        a, b = (H(o) for o in outs)
+        assert np.abs(a - b).max() <= 4e-3, step   # one fp16 step of the hidden state's values below 4
+        assert ours.cache.get_last_access_stats() == general.cache.get_last_access_stats(), step
+        assert torch.equal(ours.cache.hot_keys, general.cache.hot_keys)
+        assert torch.equal(ours.cache.warm_keys.pq_codes, general.cache.warm_keys.pq_codes)
+    assert 60 < used < 140 and ours.cache.num_cold > 0 and ours._decode.regrows + ours._decode.rebuilds > 1
+    for layer in layers:
+        layer.prefill_cache(prompt)
+    a, b = (H(layer(x, use_cache=True)) for layer in layers)
+    assert np.abs(a - b).max() <= 4e-3
