@@ -16,7 +16,7 @@
 // The Llama-3.2-1B layer's seven matrices (243 MB of fp32), torch's fp32 products
 // against this file, without the elementwise kernels around the former:
 //   1 row      88 -> 54 us (4.5 TB/s; gate and up 5.4 TB/s)
-//   1,024 rows 865 -> 343 us (363 TFLOP/s of fp32 products)
+//   1,024 rows 865 -> 317 us (393 TFLOP/s of fp32 products)
 #include "rfsn_common.h"
 #include "rfsn_internal.h"
 
@@ -443,25 +443,28 @@ linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x,
                wave * 16 + col, rows);
 }
 
-// Many rows: 128 rows of x by AN * 64 output rows per block (64 gate and 64 up
+// Many rows: 64 CT rows of x by AN * 64 output rows per block (64 gate and 64 up
 // rows under SwiGLU), two groups of 4 waves that take k runs of 32 in turn (an
 // in-block split of k: with one block or two per CU every SIMD then has two
 // waves or more), W split into its hi and lo planes on its way to LDS.
-// Bound: MFMA issue (two per product) and the LDS reads that feed it; gate and
-// up at 1,024 rows 786 TFLOP/s of issued MFMAs (175 us; 228 us before the loads
-// ran two stages ahead and the row tiles of a panel shared an XCD).
-template <int MODE, int AN, int kBK>
+// Bound: the LDS reads that feed the MFMAs (two per product), which take about as
+// long as these at AN 2, CT 2; gate and up at 1,024 rows 880 TFLOP/s of issued
+// MFMAs (156 us; 228 us before the loads ran two stages ahead and the row tiles
+// of a panel shared an XCD).
+template <int MODE, int AN, int CT, int kBK>
 __global__ void __launch_bounds__(512, 2)
 linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, int rows, int row_tiles, int panels) {
-  constexpr int kG = 2, TN = AN * 64, TS = 128, kRow = kBK / 8;
+  constexpr int kG = 2, TN = AN * 64, TS = CT * 64, kRow = kBK / 8;
   constexpr int kWv = TN * kRow, kXv = TS * kRow;                    // 16-byte units of a plane of W, of X
   constexpr int kStage = 2 * kWv + kXv;
+  // X comes from L2: where its two register sets would spill, one stage ahead is enough
+  constexpr int kXS = CT == 4 ? 1 : 2;
   constexpr int kWL = TN * kBK / 8 / 256, kXL = TS * kBK / 8 / 256;  // 8-element units a thread stages
   __shared__ uint4v smem[kG * 2 * kStage];
   __shared__ float red[8];
   __shared__ int row_max[TN];
   __shared__ float row_inv[TN];
-  static_assert(sizeof(smem) >= 256 * 32 * AN * 4, "the groups' sums fit the staging buffers");
+  static_assert(sizeof(smem) >= 256 * 16 * AN * CT * 4, "the groups' sums fit the staging buffers");
   const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave & 1, ws = wave >> 1;
   const int col = lane & 31, hf = lane >> 5;
@@ -500,7 +503,7 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
     row_max[threadIdx.x] = 0;
     row_inv[threadIdx.x] = 1.f / kScale;
   }
-  float16v acc[AN][2];
+  float16v acc[AN][CT];
   const int iters = p.k / (kBK * kG);  // the launch takes a kBK that divides k evenly
 
   auto run = [&](auto careful) {
@@ -508,7 +511,7 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < CT; ++c)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[a][c][i] = 0.f;
     // two register sets in front of the two LDS buffers: stage it + 3 is requested when
@@ -516,8 +519,14 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
     // and stored again, unread, which keeps the vmcnt waits exact and lets the
     // conversions of one stage overlap the products of another.
     float4v wv[2][kWL][2];
-    uint4v xv[2][kXL];
-    auto fetch = [&](int it, auto set) {
+    uint4v xv[kXS][kXL];
+    auto fetch_x = [&](int it, auto set) {
+      constexpr int R = decltype(set)::value % kXS;
+      const int kb = (min(it, iters - 1) * kG + grp) * kBK + kc;
+#pragma unroll
+      for (int u = 0; u < kXL; ++u) xv[R][u] = *reinterpret_cast<const uint4v*>(xrow[u] + kb);
+    };
+    auto fetch_w = [&](int it, auto set) {
       constexpr int R = decltype(set)::value;
       const int kb = (min(it, iters - 1) * kG + grp) * kBK + kc;
 #pragma unroll
@@ -525,8 +534,10 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
         wv[R][u][0] = *reinterpret_cast<const float4v*>(wrow[u] + kb);
         wv[R][u][1] = *reinterpret_cast<const float4v*>(wrow[u] + kb + 4);
       }
-#pragma unroll
-      for (int u = 0; u < kXL; ++u) xv[R][u] = *reinterpret_cast<const uint4v*>(xrow[u] + kb);
+    };
+    auto fetch = [&](int it, auto set) {  // it >= 1 with one X set
+      fetch_w(it, set);
+      fetch_x(kXS == 2 ? it : it - 1, set);
     };
     auto store = [&](auto set) {
       constexpr int R = decltype(set)::value;
@@ -540,32 +551,34 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
         s[kWv + i] = __builtin_bit_cast(uint4v, lo);
       }
 #pragma unroll
-      for (int u = 0; u < kXL; ++u) s[2 * kWv + at((u * 256 + tid) / kRow, tid % kRow)] = xv[R][u];
+      for (int u = 0; u < kXL; ++u) s[2 * kWv + at((u * 256 + tid) / kRow, tid % kRow)] = xv[R % kXS][u];
     };
     auto products = [&](auto set) {
       const uint4v* const s = sg + decltype(set)::value * kStage;
 #pragma unroll
       for (int ks = 0; ks < kBK / 16; ++ks) {
-        half8 xf[2];
+        half8 xf[CT];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          xf[c] = __builtin_bit_cast(half8, s[2 * kWv + at(ws * 64 + c * 32 + col, 2 * ks + hf)]);
+        for (int c = 0; c < CT; ++c) {
+          xf[c] = __builtin_bit_cast(half8, s[2 * kWv + at(ws * (CT * 32) + c * 32 + col, 2 * ks + hf)]);
         }
 #pragma unroll
         for (int a = 0; a < AN; ++a) {
           const int i = at(wn * AN * 32 + a * 32 + col, 2 * ks + hf);
           const half8 hi = __builtin_bit_cast(half8, s[i]), lo = __builtin_bit_cast(half8, s[kWv + i]);
 #pragma unroll
-          for (int c = 0; c < 2; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, xf[c], acc[a][c], 0, 0, 0);
+          for (int c = 0; c < CT; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, xf[c], acc[a][c], 0, 0, 0);
 #pragma unroll
-          for (int c = 0; c < 2; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, xf[c], acc[a][c], 0, 0, 0);
+          for (int c = 0; c < CT; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, xf[c], acc[a][c], 0, 0, 0);
         }
       }
     };
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
-    fetch(0, even);
-    fetch(1, odd);
+    fetch_w(0, even);
+    fetch_x(0, even);
+    fetch_w(1, odd);
+    if (kXS == 2) fetch_x(1, odd);
     store(even);
     fetch(2, even);
     __syncthreads();
@@ -600,25 +613,25 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
     }
     run(std::true_type{});
   }
-  float* m = reinterpret_cast<float*>(smem) + wave * AN * 32 * 64 + lane;
+  float* m = reinterpret_cast<float*>(smem) + wave * AN * CT * 16 * 64 + lane;
   if (grp == 1) {
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m[((a * 2 + c) * 16 + i) * 64] = acc[a][c][i];
+        for (int i = 0; i < 16; ++i) m[((a * CT + c) * 16 + i) * 64] = acc[a][c][i];
   }
   __syncthreads();
   if (grp == 1) return;
   const float* ri = row_inv + wn * AN * 32;  // the wave's staged rows (32 gate, then 32 up, under SwiGLU)
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < CT; ++c) {
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][c][i] += m[((a * 2 + c) * 16 + i) * 64];
-    const int s = s0 + ws * 64 + c * 32 + col;
+      for (int i = 0; i < 16; ++i) acc[a][c][i] += m[((a * CT + c) * 16 + i) * 64];
+    const int s = s0 + ws * (CT * 32) + c * 32 + col;
     if (MODE == kModeSwiglu) {
       write_tile<MODE>(p, acc[0][c], acc[AN - 1][c], ri, ri + 32, n0 + wn * 32, limit, s, rows, hf);
     } else {
@@ -664,14 +677,34 @@ int launch_linear(const rfsn_linear_params& p, hipStream_t s) {
       RFSN_SKINNY(4, 8);
 #undef RFSN_SKINNY
   } else {
-    const int row_tiles = (int)ceil_div(rows, 128);
-    const int panels = (int)ceil_div(limit, 64);
-    const dim3 grid((unsigned)(row_tiles * ceil_div(panels, 8) * 8));
-    if (AN == 1 && k % 128 == 0)
-      hipLaunchKernelGGL((linear_tiles_kernel<MODE, AN, AN == 1 ? 64 : 32>), grid, dim3(512), 0, s, p, x, rows,
-                         row_tiles, panels);
-    else
-      hipLaunchKernelGGL((linear_tiles_kernel<MODE, AN, 32>), grid, dim3(512), 0, s, p, x, rows, row_tiles, panels);
+    // Blocks run 256 at a time (LDS leaves one per CU).  Twice the tile costs 1.7 to
+    // 1.8 times the round, as its waves read less LDS per MFMA, and pays where it
+    // halves the rounds: gate and up at 1,024 rows 170 -> 156 us (768 rows, two
+    // rounds against three: 133 -> 143), qkv at 1,024 rows 56 -> 50 us.
+    auto blocks = [&](int out_rows, int x_rows) {
+      return ceil_div(ceil_div(limit, out_rows), 8) * 8 * ceil_div(rows, x_rows);
+    };
+#define RFSN_TILES(A, CT, BK)                                                                                          \
+  do {                                                                                                                 \
+    const int panels = (int)ceil_div(limit, MODE == kModeSwiglu ? 32 * A : 64 * A);                                    \
+    const int row_tiles = (int)ceil_div(rows, CT * 64);                                                                \
+    hipLaunchKernelGGL((linear_tiles_kernel<MODE, A, CT, BK>), dim3((unsigned)(row_tiles * ceil_div(panels, 8) * 8)),  \
+                       dim3(512), 0, s, p, x, rows, row_tiles, panels);                                                \
+  } while (0)
+    if constexpr (MODE == kModeSwiglu) {
+      if (16 * ceil_div(blocks(64, 256), 256) < 9 * ceil_div(blocks(64, 128), 256))
+        RFSN_TILES(2, 4, 32);
+      else
+        RFSN_TILES(2, 2, 32);
+    } else {
+      if (17 * ceil_div(blocks(128, 128), 256) < 10 * ceil_div(blocks(64, 128), 256))
+        RFSN_TILES(2, 2, 32);
+      else if (k % 128 == 0)
+        RFSN_TILES(1, 2, 64);
+      else
+        RFSN_TILES(1, 2, 32);
+    }
+#undef RFSN_TILES
   }
   if (MODE == kModePlain && p.head_dim) {
     const int groups = (int)ceil_div((p.n[0] + p.n[1]) / p.head_dim, kRopeHeads);

@@ -9,8 +9,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-ROWS = [1, 2, 16, 17, 33, 64, 65, 129, 200]
-SHAPES = [(64, 64), (192, 320), (640, 128), (2048, 68), (8192, 64)]  # k, n
+ROWS = [1, 2, 16, 17, 33, 64, 65, 129, 200, 520]
+SHAPES = [(64, 64), (192, 320), (640, 128), (2048, 68), (8192, 64), (128, 4100)]  # k, n (the last: larger tiles)
 
 
 def _t(a, device):
