@@ -1161,6 +1161,21 @@ __global__ void __launch_bounds__(W * 64, 1) warm_encode_fused_kernel(const Enco
 // launch runs every stage; a row's running residual stays in a float32
 // workspace [A][D] between stages (stage 0 reads the fp16 PQ residual).
 //
+// What is said here holds for rvq_keys_kernel, a key per centroid: 5 VALU
+// operations a distance beside the MFMA's share of 16 cycles per 4.
+// rvq_mfma_kernel, which serves large codebooks and few rows, keeps a key per
+// group of four centroids (the least of the lane's four distances): 7 operations
+// a group, run in the shadow of the next tile's MFMAs.  Groups within 2E + t of the
+// first key's are its candidates; the row is settled if it has one such group and
+// that group one centroid within 2E of its least (its four distances are taken again
+// from the B operand).  Other rows, up to 5 groups, take their distances
+// from the unrounded x, a wave per row, and what that leaves open (2E' = 2.5 (mfma
+// + canon)) the float64 chain.  A lane keeps four keys and the row merges its lanes'
+// sixteen: the list is complete if every lane's fourth is apart from the first.
+// 131,072 rows of 128 x 4 stages of 4,096 (550 GFLOP): 880 us -> 623, 0.88 PFLOP/s;
+// 4,000 rows: 510 -> 194.  Left: the four-centroid reads (1 KB of L2 a row and stage),
+// and MFMA, VALU and LDS phases that two waves a SIMD overlap in part only.
+//
 // Screening: a block (4 waves) holds 4 * kRvqSets * 16 rows; each wave holds
 // kRvqSets B operands of 16 rows as -fp16(x) (v_mfma_f32_16x16x32_f16: lane l
 // has row l % 16, coordinates 32 ks + 8 (l / 16) + e).  The stage's codebook
@@ -1191,6 +1206,10 @@ __global__ void __launch_bounds__(W * 64, 1) warm_encode_fused_kernel(const Enco
 constexpr int kRvqWaves = 4;
 constexpr int kRvqThreads = kRvqWaves * 64;
 constexpr int kRvqChunk = 64;          // centroid rows per LDS chunk
+constexpr int kRvqItems = 16;          // rows a wave rescores together
+constexpr int kRvqKeysCentroids = 512;  // a key per centroid up to here ...
+constexpr int64_t kRvqKeysRows = 65536;  // ... and past this many rows
+constexpr int kRvqGroups = 5;          // most candidate groups of such a row
 constexpr float kRvqPadHalfR = 1.0e38f;  // R / 2 of rows past the codebook: never a minimum
 
 template <int D>
@@ -1198,12 +1217,13 @@ struct RvqShape {
   static constexpr int KS = D / 32;               // 16x16x32 k-steps
   static constexpr int G16 = D / 8;               // 16-byte groups of a row
   static constexpr int RB = D * 2;                // row bytes
-  static constexpr int SETS = D <= 128 ? 4 : 2;   // B operands per wave
-  static constexpr int VECS = kRvqWaves * SETS * 16;
+  static constexpr int SETS = D <= 128 ? 4 : 2;   // most B operands (16 rows each) per wave
 };
 
 typedef _Float16 rh8 __attribute__((ext_vector_type(8)));
+typedef _Float16 rh4 __attribute__((ext_vector_type(4)));
 typedef float rf4 __attribute__((ext_vector_type(4)));
+typedef uint32_t ru4 __attribute__((ext_vector_type(4)));
 
 // canonical R_j = fl32(S c_j * c_j) per (stage, centroid) into r[L][Cp]
 // (rows past C: +inf): one thread per row, the row in 16-byte loads
@@ -1264,9 +1284,599 @@ __device__ __forceinline__ void fkey_insert4(float& m1, float& m2, float& m3, fl
       : "v"(k));
 }
 
-template <int D>
+// the same in single instructions, which the compiler places between MFMAs
+__device__ __forceinline__ void fkey_push4(float& m1, float& m2, float& m3, float& m4, float k) {
+  m4 = __builtin_amdgcn_fmed3f(m3, m4, k);
+  m3 = __builtin_amdgcn_fmed3f(m2, m3, k);
+  m2 = __builtin_amdgcn_fmed3f(m1, m2, k);
+  asm("v_min_f32_e32 %0, %0, %1" : "+v"(m1) : "v"(k));
+}
+
+// v of the lane that the DPP control names, within 16 lanes
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+
+template <int D, int SETS>
 __global__ void __launch_bounds__(kRvqThreads) __attribute__((amdgpu_waves_per_eu(2)))
 rvq_mfma_kernel(const uint16_t* __restrict__ resid, int64_t ld, const int32_t* __restrict__ offsets,
+                int64_t active, const uint16_t* __restrict__ cb, int L, int C, int Cp, int F,
+                const float* __restrict__ rr, const float* __restrict__ rmax_all, float* __restrict__ run,
+                uint16_t* __restrict__ codes) {
+  using S = RvqShape<D>;
+  constexpr int KS = S::KS, G16 = S::G16, RB = S::RB;
+  __shared__ __align__(16) uint8_t tab[2][kRvqChunk * RB];
+  __shared__ __align__(16) float rs[2][kRvqChunk];
+  __shared__ float xsc[kRvqWaves][D];  // one row's coordinates for the wave's float64 scans
+  __shared__ int pitem[kRvqWaves][SETS * 16][kRvqGroups];  // rows to rescore: their groups
+  __shared__ int pslot[kRvqWaves][SETS * 16];          // item -> row (16 s + vi) and group count
+  __shared__ int pcode[kRvqWaves][SETS * 16];          // item -> its 2E', then its code or -1
+  __shared__ double pres[kRvqWaves][kRvqItems][1 + 4 * kRvqGroups];  // L, then X of each candidate
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int vi = lane & 15, g = lane >> 4;
+  const int64_t v0 = (int64_t)(blockIdx.x * kRvqWaves + wave) * (SETS * 16);
+  int64_t vid[SETS];
+  bool live[SETS];
+  int prow[SETS];  // the row of the PQ residual
+#pragma unroll
+  for (int s = 0; s < SETS; ++s) {
+    vid[s] = v0 + 16 * s + vi;
+    live[s] = vid[s] < active;
+    // lanes past the last row follow it: they load and store nothing of their own
+    vid[s] = live[s] ? vid[s] : active - 1;
+    prow[s] = offsets[vid[s]];
+  }
+  const int fmask = (1 << F) - 1;
+  const int keep = ~fmask;  // key bits kept from z (in a VGPR: the key build's other operand is an SGPR)
+  int keepv;
+  asm("v_mov_b32 %0, %1" : "=v"(keepv) : "s"(keep));
+  float ninf;  // -inf, unknown to the compiler: med3 with it is a plain v_med3, no canonicalising min
+  asm("v_mov_b32 %0, 0xff800000" : "=v"(ninf));
+
+  // the row's coordinate u at the current stage: the fp16 PQ residual at stage 0, then the workspace
+  auto x_at = [&](int64_t v, int layer, int u) -> float {
+    return layer == 0 ? h2f(resid[(int64_t)offsets[v] * ld + u]) : run[v * D + u];
+  };
+  // coordinates k0 .. k0 + 7 of a row: the PQ residual's (row of resid) or the workspace's (row v);
+  // which one is known when it is compiled, so that no load stands behind a branch
+  auto load_x8 = [&](auto first, int prow, int64_t v, int k0, float (&x)[8]) {
+    if constexpr (decltype(first)::value) {
+      const rh8 h = *reinterpret_cast<const rh8*>(resid + (int64_t)prow * ld + k0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (float)h[e];
+    } else {
+      const rf4 a = *reinterpret_cast<const rf4*>(run + v * D + k0);
+      const rf4 b = *reinterpret_cast<const rf4*>(run + v * D + k0 + 4);
+      x[0] = a[0]; x[1] = a[1]; x[2] = a[2]; x[3] = a[3];
+      x[4] = b[0]; x[5] = b[1]; x[6] = b[2]; x[7] = b[3];
+    }
+  };
+
+  rh8 b[SETS][KS];
+  float lsq[SETS], esq[SETS];  // |x|^2 and |x - fp16(x)|^2 (the lane's share, then the row's)
+  bool fin[SETS];
+  // the B operand -fp16(x) of 8 coordinates, with their shares of |x|^2 and of the rounding error
+  auto to_b = [](const float (&x)[8], rh8& bo, float& l2, float& e2, bool& ok) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const _Float16 h = (_Float16)x[e];
+      bo[e] = -h;
+      const float d = x[e] - (float)h;  // exact in float32
+      l2 = __builtin_fmaf(x[e], x[e], l2);
+      e2 = __builtin_fmaf(d, d, e2);
+      ok = ok && fabsf(x[e]) <= 65504.0f;
+    }
+  };
+  // B operands and the screening L of each row at stage 0
+#pragma unroll
+  for (int s = 0; s < SETS; ++s) {
+    float l2 = 0.0f, e2 = 0.0f;
+    bool ok = true;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      float x[8];
+      load_x8(std::true_type{}, prow[s], vid[s], 32 * ks + 8 * g, x);
+      to_b(x, b[s][ks], l2, e2, ok);
+    }
+    lsq[s] = l2;
+    esq[s] = e2;
+    fin[s] = ok;
+  }
+  auto quad_sum = [&](float v) {  // sum over the row's four lanes l, l ^ 16, l ^ 32, l ^ 48
+    v += __builtin_bit_cast(float, lane_xor16(__builtin_bit_cast(int, v)));
+    return v + __builtin_bit_cast(float, lane_xor32(__builtin_bit_cast(int, v), 4 * (lane ^ 32)));
+  };
+  auto quad_all = [&](bool p) {
+    int v = p ? 1 : 0;
+    v &= lane_xor16(v);
+    return (v & lane_xor32(v, 4 * (lane ^ 32))) != 0;
+  };
+
+  const int nchunks = Cp / kRvqChunk;
+  constexpr int kLoads = kRvqChunk * G16 / kRvqThreads;  // 16-byte staging loads per thread and chunk
+  static_assert(kRvqChunk * G16 % kRvqThreads == 0, "staging loads per thread");
+  // 16-byte groups are XOR-ed with the row's low bits: 16 rows hit the 64 banks evenly, and a
+  // lane's groups lie alike in every tile of 16 rows
+  constexpr int kSwz = (G16 < 16 ? G16 : 16) - 1;
+  constexpr int kTiles = kRvqChunk / 16;
+  uint32_t aoff[KS];  // the lane's A operands in a tile
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) aoff[ks] = vi * RB + 16 * ((4 * ks + g) ^ (vi & kSwz));
+
+  for (int layer = 0; layer < L; ++layer) {
+    const uint16_t* cbl = cb + (size_t)layer * C * D;
+    const float* rl = rr + (size_t)layer * Cp;
+    const float rmax = rmax_all[layer];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      lsq[s] = quad_sum(lsq[s]);
+      esq[s] = quad_sum(esq[s]);
+      fin[s] = quad_all(fin[s]);
+    }
+    // ---- staging of chunk c into buffer c & 1: loads, then stores
+    ru4 stg[kLoads];
+    float rstg;
+    auto stage_load = [&](int c) {
+#pragma unroll
+      for (int it = 0; it < kLoads; ++it) {
+        const int q = tid + kRvqThreads * it;
+        const int row = q / G16, grp = q % G16;
+        const int j = min(c * kRvqChunk + row, C - 1);  // rows past the codebook: their R / 2 keeps them out
+        stg[it] = *reinterpret_cast<const ru4*>(cbl + (size_t)j * D + 8 * grp);
+      }
+      rstg = rl[c * kRvqChunk + (tid & (kRvqChunk - 1))];
+    };
+    auto stage_store = [&](int c) {
+      uint8_t* tb = tab[c & 1];
+#pragma unroll
+      for (int it = 0; it < kLoads; ++it) {
+        const int q = tid + kRvqThreads * it;
+        const int row = q / G16, grp = q % G16;
+        *reinterpret_cast<ru4*>(tb + row * RB + 16 * (grp ^ (row & kSwz))) = stg[it];
+      }
+      rs[c & 1][tid & (kRvqChunk - 1)] = fminf(0.5f * rstg, kRvqPadHalfR);  // the waves write the same
+    };
+    __syncthreads();  // the previous stage's last chunk is no longer read
+    stage_load(0);
+    stage_store(0);
+    __syncthreads();
+
+    float m1[SETS], m2[SETS], m3[SETS], m4[SETS];
+    const float nokey = __builtin_inff();
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) m1[s] = m2[s] = m3[s] = m4[s] = nokey;
+    // the least of the lane's four distances stands for their group: the compiler
+    // sees, and pads, the first read of the MFMA result; the rest depends on it
+    auto filter = [&](const rf4 (&acc)[SETS], int base) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        const float z0 = acc[s][0], z1 = acc[s][1], z2 = acc[s][2], z3 = acc[s][3];
+        float z = __builtin_amdgcn_fmed3f(z0, z1, ninf);
+        asm("v_min3_f32 %0, %0, %1, %2" : "+v"(z) : "v"(z2), "v"(z3));
+        const float key = __builtin_bit_cast(float, (__builtin_bit_cast(int, z) & keepv) | base);
+        fkey_push4(m1[s], m2[s], m3[s], m4[s], key);
+      }
+    };
+    // a tile's distances are filtered while the next tile's products run
+    rf4 acc[2][SETS];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) acc[1][s] = rf4{kRvqPadHalfR, kRvqPadHalfR, kRvqPadHalfR, kRvqPadHalfR};
+#pragma unroll 1
+    for (int c = 0; c < nchunks; ++c) {
+      stage_load(min(c + 1, nchunks - 1));  // after the last chunk: read again, never used
+      const uint8_t* tb = tab[c & 1];
+      const float* rb = rs[c & 1] + 4 * g;
+#pragma unroll
+      for (int tile = 0; tile < kTiles; ++tile) {
+        rh8 a[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) a[ks] = *reinterpret_cast<const rh8*>(tb + aoff[ks] + tile * 16 * RB);
+        const rf4 rinit = *reinterpret_cast<const rf4*>(rb + tile * 16);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int s = 0; s < SETS; ++s)
+            acc[tile & 1][s] =
+                __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks], b[s][ks], ks ? acc[tile & 1][s] : rinit, 0, 0, 0);
+        // the group's order 4 T (the lane's g is added after the scan), in an SGPR
+        filter(acc[~tile & 1], __builtin_amdgcn_readfirstlane(max(4 * (c * kTiles + tile - 1), 0)));
+#ifdef SGB
+#pragma unroll
+        for (int i = 0; i < SETS * KS; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, SGB, 0);
+        }
+#endif
+      }
+      stage_store(c + 1);
+      __syncthreads();
+    }
+    filter(acc[(kTiles - 1) & 1], __builtin_amdgcn_readfirstlane(4 * (nchunks * kTiles - 1)));
+
+    // ---- merge the row's four lanes: group 4 T + g holds centroids 16 T + 4 g .. + 3
+    auto widen = [&](float k) { return __builtin_bit_cast(float, __builtin_bit_cast(int, k) | g); };
+    const float Cn = sqrtf(rmax) * 1.0001f;
+    int code[SETS];
+    int how[SETS];                        // 0 settled, 1 rescore the groups, 2 full scan
+    int ng[SETS];                         // candidate groups
+    int jg[SETS][kRvqGroups];             // their first centroids
+    float slack[SETS], fine[SETS];        // twice the error of a distance: from the B operand, from x
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      // the row's six smallest keys of its lanes' sixteen
+      const float own4 = m4[s];
+      float p[6] = {widen(m1[s]), widen(m2[s]), widen(m3[s]), widen(m4[s]), nokey, nokey};
+      auto merge_from = [&](auto&& other) {
+        float o[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) o[k] = __builtin_bit_cast(float, other(__builtin_bit_cast(int, p[k])));
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          p[5] = __builtin_amdgcn_fmed3f(p[4], p[5], o[k]);
+          p[4] = __builtin_amdgcn_fmed3f(p[3], p[4], o[k]);
+          fkey_push4(p[0], p[1], p[2], p[3], o[k]);
+        }
+      };
+      merge_from([](int v) { return lane_xor16(v); });
+      const int x32 = 4 * (lane ^ 32);
+      merge_from([&](int v) { return lane_xor32(v, x32); });
+      const float xn = sqrtf(lsq[s]) * 1.0001f;
+      const float split = sqrtf(esq[s]) * 1.0001f * Cn;  // |(x - fp16(x)) . c_j| <= |x - fp16(x)| Cn
+      const float mf = (float)(D + 2) * 0x1p-24f * (xn * Cn + 0.5f * rmax);
+      const float canon = 0x1p-21f * (lsq[s] + rmax);
+      const float E = 1.25f * (split + mf + canon) + 0x1p-100f;
+      const float tq = __builtin_bit_cast(float, (127 + F - 22) << 23);  // 2^(F - 22)
+      const bool safe = fin[s] && lsq[s] <= 1.0e30f && rmax <= 1.0e30f && C >= 3;
+      // candidate groups: the keys within 2E + t of the first
+      auto apart = [&](float a, float b) { return b - a > 2.0f * E + tq * (fabsf(a) + fabsf(b)); };
+      // a lane's unlisted groups lie past its fourth key: that one has to be apart too
+      const bool listed = quad_all(apart(p[0], own4)) && apart(p[0], p[5]);
+      ng[s] = apart(p[0], p[1]) ? 1 : apart(p[0], p[2]) ? 2 : apart(p[0], p[3]) ? 3 : apart(p[0], p[4]) ? 4 : 5;
+      how[s] = !live[s] ? 0 : !safe || !listed ? 2 : ng[s] == 1 ? 0 : 1;
+      slack[s] = 2.0f * E;
+      fine[s] = 2.5f * (mf + canon) + 0x1p-99f;
+#pragma unroll
+      for (int k = 0; k < kRvqGroups; ++k) jg[s][k] = 4 * (__builtin_bit_cast(int, p[k]) & fmask);
+    }
+    // ---- the first group's four centroids again, against the B operand: a lane sums its
+    // coordinates of each; the loads of a unit (KQ k-steps of a set) run ahead by one unit
+    float dot[SETS][4];
+    constexpr int KQ = KS < 4 ? KS : 4, kUnits = SETS * (KS / KQ);
+    rh8 cw[2][KQ][4];
+    auto unit_load = [&](int n) {
+      const int s = n / (KS / KQ), k0 = n % (KS / KQ) * KQ;
+#pragma unroll
+      for (int q = 0; q < KQ; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          cw[n & 1][q][i] =
+              *reinterpret_cast<const rh8*>(cbl + (size_t)min(jg[s][0] + i, C - 1) * D + 32 * (k0 + q) + 8 * g);
+    };
+    unit_load(0);
+#pragma unroll
+    for (int n = 0; n < kUnits; ++n) {
+      const int s = n / (KS / KQ), k0 = n % (KS / KQ) * KQ;
+      if (n + 1 < kUnits) unit_load(n + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 == 0) dot[s][0] = dot[s][1] = dot[s][2] = dot[s][3] = 0.0f;
+#pragma unroll
+      for (int q = 0; q < KQ; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            dot[s][i] = __builtin_fmaf((float)b[s][k0 + q][e], (float)cw[n & 1][q][i][e], dot[s][i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      float z[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // rows past the codebook: +inf
+        z[i] = 0.5f * rl[min(jg[s][0] + i, Cp - 1)] + quad_sum(dot[s][i]);
+      const float cut = fminf(fminf(z[0], z[1]), fminf(z[2], z[3])) + slack[s];
+      int n = 0;
+      code[s] = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (z[i] <= cut) {
+          code[s] = jg[s][0] + i;
+          ++n;
+        }
+      }
+      if (how[s] == 0 && live[s] && n != 1) how[s] = 1;
+    }
+    // ---- rows with more candidates: listed, then every candidate group's distances with
+    // the unrounded x, a wave per row (16 lanes a centroid), two rows' loads in flight;
+    // one centroid within 2E' of the least settles the row
+    int nitems = 0;
+    int myitem[SETS];
+    auto list_rows = [&]() {
+      nitems = 0;
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        const uint64_t want = __builtin_amdgcn_ballot_w64(g == 0 && how[s] == 1);
+        // every lane of row vi takes the row's rank among the set's wanting rows
+        const int rank = __builtin_popcountll(want & ((1ull << vi) - 1));
+        myitem[s] = ((want >> vi) & 1) ? nitems + rank : -1;
+        if (g == 0 && myitem[s] >= 0) {
+#pragma unroll
+          for (int k = 0; k < kRvqGroups; ++k) pitem[wave][myitem[s]][k] = jg[s][k];
+          pslot[wave][myitem[s]] = 16 * s + vi + (ng[s] << 8);
+          pcode[wave][myitem[s]] = __builtin_bit_cast(int, fine[s]);
+        }
+        nitems += __builtin_popcountll(want);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    list_rows();
+    if (nitems) {  // uniform
+      auto settle = [&](auto first) {
+        constexpr int CL = D / 16, IF = D <= 128 ? 2 : 1;
+        const int k0 = CL * vi;
+#pragma unroll 1
+        for (int i0 = 0; i0 < nitems; i0 += IF) {
+          rh4 cw[IF][kRvqGroups][CL / 4];
+          float x[IF][CL], hr[IF][kRvqGroups];
+          int slot[IF], gj[IF][kRvqGroups];
+          float tol[IF];
+#pragma unroll
+          for (int h = 0; h < IF; ++h) {
+            const int it = min(i0 + h, nitems - 1);
+            slot[h] = pslot[wave][it];
+            tol[h] = __builtin_bit_cast(float, pcode[wave][it]);
+            const int64_t v = v0 + (slot[h] & 255);
+            if constexpr (decltype(first)::value) {
+              const uint16_t* xr = resid + (int64_t)offsets[v] * ld + k0;
+#pragma unroll
+              for (int q = 0; q < CL / 4; ++q) {
+                const rh4 t = reinterpret_cast<const rh4*>(xr)[q];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[h][4 * q + e] = (float)t[e];
+              }
+            } else {
+#pragma unroll
+              for (int q = 0; q < CL / 4; ++q) {
+                const rf4 t = reinterpret_cast<const rf4*>(run + v * D + k0)[q];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[h][4 * q + e] = t[e];
+              }
+            }
+#pragma unroll
+            for (int k = 0; k < kRvqGroups; ++k) {
+              gj[h][k] = pitem[wave][it][k];
+              const int j = gj[h][k] + g;
+              hr[h][k] = 0.5f * rl[min(j, Cp - 1)];  // rows past the codebook: +inf
+              const uint16_t* cr = cbl + (size_t)min(j, C - 1) * D + k0;
+#pragma unroll
+              for (int q = 0; q < CL / 4; ++q) cw[h][k][q] = reinterpret_cast<const rh4*>(cr)[q];
+            }
+          }
+#pragma unroll
+          for (int h = 0; h < IF; ++h) {
+            float z[kRvqGroups], least = __builtin_inff();
+#pragma unroll
+            for (int k = 0; k < kRvqGroups; ++k) {
+              float d = 0.0f;
+#pragma unroll
+              for (int e = 0; e < CL; ++e) d = __builtin_fmaf(x[h][e], (float)cw[h][k][e / 4][e % 4], d);
+              d += dpp_f32<0xB1>(d);   // lane ^ 1
+              d += dpp_f32<0x4E>(d);   // lane ^ 2
+              d += dpp_f32<0x141>(d);  // mirrored in 8 lanes
+              d += dpp_f32<0x140>(d);  // mirrored in 16 lanes
+              z[k] = k < (slot[h] >> 8) ? hr[h][k] - d : __builtin_inff();
+              least = fminf(least, z[k]);
+            }
+            least = fminf(least, __builtin_bit_cast(float, lane_xor16(__builtin_bit_cast(int, least))));
+            least = fminf(least, __builtin_bit_cast(float, lane_xor32(__builtin_bit_cast(int, least), 4 * (lane ^ 32))));
+            int n = 0, found = 0;
+#pragma unroll
+            for (int k = 0; k < kRvqGroups; ++k) {
+              const uint64_t in = __builtin_amdgcn_ballot_w64(vi == 0 && z[k] <= least + tol[h]);
+              n += __builtin_popcountll(in);
+              if (in) found = gj[h][k] + (__builtin_ctzll(in) >> 4);
+            }
+            if (lane == 0 && i0 + h < nitems) pcode[wave][i0 + h] = n == 1 ? found : -1;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+      };
+      if (layer == 0)
+        settle(std::true_type{});
+      else
+        settle(std::false_type{});
+      bool left = false;
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        if (myitem[s] >= 0) {
+          const int found = pcode[wave][myitem[s]];
+          if (found >= 0) {
+            code[s] = found;
+            how[s] = 0;
+          }
+        }
+        left = left || how[s] == 1;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();  // the list is rewritten
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      nitems = 0;
+      if (__builtin_amdgcn_ballot_w64(left)) list_rows();  // uniform
+    }
+    // ---- rows still open (centroids equal or nearly so): float64 sums in coordinate
+    // order (L, then X of each of the groups' centroids), spread over the wave's lanes
+    // as independent units, then each row picks its code
+    {
+#pragma unroll 1
+      for (int i0 = 0; i0 < nitems; i0 += kRvqItems) {  // uniform
+        const int batch = min(nitems - i0, kRvqItems);
+        auto sums = [&](auto first) {
+#pragma unroll 1
+          for (int u = lane; u < 32 * batch; u += 64) {
+            const int it = u >> 5, comp = u & 31;
+            const int slot = pslot[wave][i0 + it];
+            if (comp > 4 * (slot >> 8)) continue;
+            const int64_t v = v0 + (slot & 255);
+            const int j = comp == 0 ? 0 : min(pitem[wave][i0 + it][(comp - 1) >> 2] + ((comp - 1) & 3), C - 1);
+            const rh8* crow = reinterpret_cast<const rh8*>(cbl + (size_t)j * D);
+            const int xrow = offsets[v];
+            double acc = 0.0;
+#pragma unroll 4
+            for (int q = 0; q < D / 8; ++q) {
+              float x8[8];
+              load_x8(first, xrow, v, 8 * q, x8);
+              const rh8 w = crow[q];  // unused for L
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const double xu = (double)x8[e];
+                acc = __builtin_fma(xu, comp == 0 ? xu : (double)(float)w[e], acc);
+              }
+            }
+            pres[wave][it][comp] = acc;
+          }
+        };
+        if (layer == 0)
+          sums(std::true_type{});
+        else
+          sums(std::false_type{});
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) {
+          const int it = myitem[s] - i0;
+          if (it < 0 || it >= batch) continue;
+          const float Lc = (float)pres[wave][it][0];
+          float bd = __builtin_inff();
+          for (int k = 0; k < 4 * ng[s]; ++k) {  // the least, the lower index of equals
+            const int j = pitem[wave][myitem[s]][k >> 2] + (k & 3);
+            const float d = __fadd_rn(__fsub_rn(Lc, 2.0f * (float)pres[wave][it][1 + k]), rl[j]);
+            if (d < bd || (d == bd && j < code[s])) {
+              bd = d;
+              code[s] = j;
+            }
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // the sums are rewritten by the next batch, the items at the next stage
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+    // ---- rows left uncertain: the canonical scan over all C, one row at a time
+    // across the wave (lane j scans centroids j, j + 64, ...)
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      uint64_t todo = __builtin_amdgcn_ballot_w64(g == 0 && live[s] && how[s] == 2);
+      while (todo) {  // uniform
+        const int r0 = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int64_t v = v0 + 16 * s + r0;
+        for (int u = lane; u < D; u += 64) xsc[wave][u] = x_at(v, layer, u);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        double lacc = 0.0;
+        for (int u = 0; u < D; ++u) {
+          const double xu = (double)xsc[wave][u];
+          lacc = __builtin_fma(xu, xu, lacc);
+        }
+        const float Lc = (float)lacc;
+        float best = __builtin_inff();
+        int bi = 0x7fffffff;
+        for (int j = lane; j < C; j += 64) {
+          const uint4* cj = reinterpret_cast<const uint4*>(cbl + (size_t)j * D);
+          double xacc = 0.0;
+#pragma unroll 4
+          for (int q = 0; q < D / 8; ++q) {  // the row's loads issued together
+            const uint4 w = cj[q];
+            const uint32_t pw[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              xacc = __builtin_fma((double)xsc[wave][8 * q + e], (double)h2f((uint16_t)(pw[e >> 1] >> (16 * (e & 1)))),
+                                   xacc);
+          }
+          const float dist = __fadd_rn(__fsub_rn(Lc, 2.0f * (float)xacc), rl[j]);
+          if (dist < best) {  // ascending j per lane: first min kept
+            best = dist;
+            bi = j;
+          }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+          const float ob = __shfl_xor(best, o, 64);
+          const int oi = __shfl_xor(bi, o, 64);
+          if (ob < best || (ob == best && oi < bi)) {
+            best = ob;
+            bi = oi;
+          }
+        }
+        if (bi == 0x7fffffff) bi = 0;  // no finite distance: index 0, as the reference's merge leaves it
+        if (vi == r0) code[s] = bi;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // xsc is rewritten by the next row
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+    // ---- codes, then the next stage's running residual fl32(run - c) and B operands:
+    // the loads of UP sets are in flight together
+#pragma unroll
+    for (int s = 0; s < SETS; ++s)
+      if (live[s] && g == 0) codes[vid[s] * L + layer] = (uint16_t)code[s];
+    if (layer + 1 == L) break;
+    constexpr int UP = SETS < 2 || KS > 4 ? 1 : 2;
+    auto next_rows = [&](auto first) {
+#pragma unroll
+      for (int s0 = 0; s0 < SETS; s0 += UP) {
+        float x[UP][KS][8];
+        rh8 cw[UP][KS];
+#pragma unroll
+        for (int h = 0; h < UP; ++h) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            cw[h][ks] = *reinterpret_cast<const rh8*>(cbl + (size_t)min(code[s0 + h], C - 1) * D + 32 * ks + 8 * g);
+            load_x8(first, prow[s0 + h], vid[s0 + h], 32 * ks + 8 * g, x[h][ks]);
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < UP; ++h) {
+          const int s = s0 + h;
+          float l2 = 0.0f, e2 = 0.0f;
+          bool ok = true;
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[h][ks][e] = __fsub_rn(x[h][ks][e], (float)cw[h][ks][e]);
+            to_b(x[h][ks], b[s][ks], l2, e2, ok);
+          }
+          if (live[s]) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+              float* out = run + vid[s] * D + 32 * ks + 8 * g;
+              *reinterpret_cast<rf4*>(out) = rf4{x[h][ks][0], x[h][ks][1], x[h][ks][2], x[h][ks][3]};
+              *reinterpret_cast<rf4*>(out + 4) = rf4{x[h][ks][4], x[h][ks][5], x[h][ks][6], x[h][ks][7]};
+            }
+          }
+          lsq[s] = l2;
+          esq[s] = e2;
+          fin[s] = ok;
+        }
+      }
+    };
+    if (layer == 0)
+      next_rows(std::true_type{});
+    else
+      next_rows(std::false_type{});
+  }
+}
+
+template <int D>
+__global__ void __launch_bounds__(kRvqThreads) __attribute__((amdgpu_waves_per_eu(2)))
+rvq_keys_kernel(const uint16_t* __restrict__ resid, int64_t ld, const int32_t* __restrict__ offsets,
                 int64_t active, const uint16_t* __restrict__ cb, int L, int C, int Cp, int F,
                 const float* __restrict__ rr, const float* __restrict__ rmax_all, float* __restrict__ run,
                 uint16_t* __restrict__ codes) {
@@ -1280,7 +1890,7 @@ rvq_mfma_kernel(const uint16_t* __restrict__ resid, int64_t ld, const int32_t* _
   __shared__ double pres[kRvqWaves][SETS * 16][4];   // L, then X of each candidate
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int vi = lane & 15, g = lane >> 4;
-  const int64_t v0 = (int64_t)blockIdx.x * S::VECS + wave * (SETS * 16);
+  const int64_t v0 = (int64_t)blockIdx.x * kRvqWaves * SETS * 16 + wave * (SETS * 16);
   int64_t vid[SETS];
   bool live[SETS];
 #pragma unroll
@@ -1666,7 +2276,7 @@ int launch_rvq_mfma(const void* resid, int64_t ld, const int32_t* offsets, int64
                     int C, uint16_t* codes, void* ws, hipStream_t s) {
   const int Cp = (C + kRvqChunk - 1) / kRvqChunk * kRvqChunk;
   int F = 0;
-  while ((1 << F) < Cp) ++F;
+  while ((4 << F) < Cp) ++F;
   const auto up = [](int64_t n) { return (size_t)((n + 255) / 256 * 256); };
   float* r = (float*)ws;
   float* rmax = (float*)((uint8_t*)ws + up(4 * L * (int64_t)Cp));
@@ -1674,9 +2284,46 @@ int launch_rvq_mfma(const void* resid, int64_t ld, const int32_t* offsets, int64
   hipLaunchKernelGGL(rvq_norms_kernel<D>, dim3((unsigned)ceil_div(Cp, 256), (unsigned)L), dim3(256), 0, s,
                      (const uint16_t*)cb, C, Cp, r);
   hipLaunchKernelGGL(rvq_rmax_kernel, dim3(L), dim3(256), 0, s, (const float*)r, C, Cp, rmax);
-  const int64_t blocks = ceil_div(active, (int64_t)RvqShape<D>::VECS);
-  hipLaunchKernelGGL(rvq_mfma_kernel<D>, dim3((unsigned)blocks), dim3(kRvqThreads), 0, s, (const uint16_t*)resid, ld,
-                     offsets, active, (const uint16_t*)cb, L, C, Cp, F, (const float*)r, (const float*)rmax, run, codes);
+  // Which kernel: reading four centroids of every row again costs the grouped screening about
+  // 1 KB of L2 traffic a row and stage, which small codebooks over many rows do not win back
+  // (2 stages of 256, D 128: 81 us by keys against 102 at 131,072 rows, 66 against 59 at
+  // 65,536; of 512: 100 against 122 at 131,072; of 1,024: 151 against 147).
+  if (C <= kRvqKeysCentroids && active > kRvqKeysRows) {
+    int F1 = 0;
+    while ((1 << F1) < Cp) ++F1;
+    hipLaunchKernelGGL(rvq_keys_kernel<D>,
+                       dim3((unsigned)ceil_div(active, (int64_t)kRvqWaves * RvqShape<D>::SETS * 16)), dim3(kRvqThreads),
+                       0, s, (const uint16_t*)resid, ld, offsets, active, (const uint16_t*)cb, L, C, Cp, F1,
+                       (const float*)r, (const float*)rmax, run, codes);
+    return check_launch("rvq_encode_full");
+  }
+  // Sets per wave.  Two blocks run on a CU at a time: 256 blocks of 1, 2 or 4 sets take about
+  // 11, 14, 21 units and 512 of them 14, 19, 31 (2 stages of 4,096, D 128: 109, 121, 198 us at
+  // 4,000 rows; 266, 184, 216 at 65,536; 488, 340, 312 at 131,072): the sets whose rounds cost least.
+  int sets = 1;
+  int64_t least = INT64_MAX;
+  const auto consider = [&](int n, int one, int two) {
+    const int64_t blocks = ceil_div(active, (int64_t)kRvqWaves * n * 16), rem = blocks % 512;
+    const int64_t cost = blocks / 512 * two + (rem == 0 ? 0 : rem <= 256 ? one : two);
+    if (cost <= least) {
+      least = cost;
+      sets = n;
+    }
+  };
+  consider(1, 11, 14);
+  consider(2, 14, 19);
+  if (RvqShape<D>::SETS == 4) consider(4, 21, 31);
+#define RFSN_RVQ(SETS)                                                                                                 \
+  hipLaunchKernelGGL((rvq_mfma_kernel<D, SETS>), dim3((unsigned)ceil_div(active, (int64_t)kRvqWaves * SETS * 16)),     \
+                     dim3(kRvqThreads), 0, s, (const uint16_t*)resid, ld, offsets, active, (const uint16_t*)cb, L, C,  \
+                     Cp, F, (const float*)r, (const float*)rmax, run, codes)
+  if (sets == 1)
+    RFSN_RVQ(1);
+  else if (sets == 2)
+    RFSN_RVQ(2);
+  else
+    RFSN_RVQ(RvqShape<D>::SETS);
+#undef RFSN_RVQ
   return check_launch("rvq_encode_full");
 }
 
