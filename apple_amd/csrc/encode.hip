@@ -1207,8 +1207,6 @@ constexpr int kRvqWaves = 4;
 constexpr int kRvqThreads = kRvqWaves * 64;
 constexpr int kRvqChunk = 64;          // centroid rows per LDS chunk
 constexpr int kRvqItems = 16;          // rows a wave rescores together
-constexpr int kRvqKeysCentroids = 512;  // a key per centroid up to here ...
-constexpr int64_t kRvqKeysRows = 65536;  // ... and past this many rows
 constexpr int kRvqGroups = 5;          // most candidate groups of such a row
 constexpr float kRvqPadHalfR = 1.0e38f;  // R / 2 of rows past the codebook: never a minimum
 
@@ -2285,10 +2283,14 @@ int launch_rvq_mfma(const void* resid, int64_t ld, const int32_t* offsets, int64
                      (const uint16_t*)cb, C, Cp, r);
   hipLaunchKernelGGL(rvq_rmax_kernel, dim3(L), dim3(256), 0, s, (const float*)r, C, Cp, rmax);
   // Which kernel: reading four centroids of every row again costs the grouped screening about
-  // 1 KB of L2 traffic a row and stage, which small codebooks over many rows do not win back
-  // (2 stages of 256, D 128: 81 us by keys against 102 at 131,072 rows, 66 against 59 at
-  // 65,536; of 512: 100 against 122 at 131,072; of 1,024: 151 against 147).
-  if (C <= kRvqKeysCentroids && active > kRvqKeysRows) {
+  // 8 D bytes of L2 traffic a row and stage, which small codebooks over many rows do not win
+  // back.  2 stages, us by groups / by keys: 256 centroids, D 128: 60 / 66 at 65,536 rows, 102 /
+  // 81 at 131,072; 512: 67 / 78, 122 / 100; 1,024: 139 / 137 at 80,000, 145 / 131 at 100,000,
+  // and at D 64 80 / 92; 2,048: 201 / 272 at 131,072.  256 at D 256: 71 / 82 at 32,768, 101 /
+  // 86 at 33,000.
+  const bool keys = (active > 65536 && (C <= 512 || (D >= 128 && C <= 1024 && active > 98304))) ||
+                    (D == 256 && C <= 256 && active > 32768);
+  if (keys) {
     int F1 = 0;
     while ((1 << F1) < Cp) ++F1;
     hipLaunchKernelGGL(rvq_keys_kernel<D>,
