@@ -1479,13 +1479,6 @@ rvq_mfma_kernel(const uint16_t* __restrict__ resid, int64_t ld, const int32_t* _
                 __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks], b[s][ks], ks ? acc[tile & 1][s] : rinit, 0, 0, 0);
         // the group's order 4 T (the lane's g is added after the scan), in an SGPR
         filter(acc[~tile & 1], __builtin_amdgcn_readfirstlane(max(4 * (c * kTiles + tile - 1), 0)));
-#ifdef SGB
-#pragma unroll
-        for (int i = 0; i < SETS * KS; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, SGB, 0);
-        }
-#endif
       }
       stage_store(c + 1);
       __syncthreads();
