@@ -93,8 +93,10 @@ def _rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float) -> to
 def _unwatched(x: torch.Tensor) -> bool:
     """Whether a call on ``x`` may pass torch's operators by: nothing records
     gradients of it (reverse or forward mode), maps, traces or compiles it,
-    intercepts its operators or casts them, and it is a plain tensor."""
-    return (type(x) is torch.Tensor and not (x.requires_grad and torch.is_grad_enabled())
+    intercepts its operators or casts them, and it is a plain tensor (or
+    parameter).  A tensor that torch.func maps or differentiates has a plain
+    type and no address: it is told by its wrapper, before anything reads it."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
             and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
             and torch._C._get_tracing_state() is None and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._len_torch_function_stack() == 0 and torch.autograd.forward_ad._current_level < 0
@@ -102,9 +104,11 @@ def _unwatched(x: torch.Tensor) -> bool:
 
 
 def _plain_weight(w: torch.Tensor, device: torch.device) -> bool:
-    """A weight the projection kernel reads as it is: fp32, contiguous, aligned, on the device, not trained."""
-    return (w.dtype is torch.float32 and w.device == device and w.is_contiguous() and w.data_ptr() % 16 == 0
-            and not (w.requires_grad and torch.is_grad_enabled()) and type(w) in (torch.nn.Parameter, torch.Tensor))
+    """A weight the projection kernel reads as it is: fp32, contiguous, aligned, on the device, and nothing
+    watches it (``_unwatched``, whose checks of the call itself the caller has made for its input)."""
+    return (type(w) in (torch.nn.Parameter, torch.Tensor) and not torch._C._functorch.is_functorch_wrapped_tensor(w)
+            and not (w.requires_grad and torch.is_grad_enabled()) and w.dtype is torch.float32 and w.device == device
+            and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
 class RFSNDecoderLayerMLX(torch.nn.Module):
