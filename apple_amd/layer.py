@@ -354,12 +354,21 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
                          for t in (cos, sin))
         return rope_cos_sin(pid, self.head_dim, self.rope_theta, self.rope_scaling)
 
-    def _native(self, h16: torch.Tensor) -> bool:
+    def _given_tables(self, seq_len: int, position_embeddings, position_ids) -> Optional[Tuple]:
+        """The call's rotary tables where the caller or ``rotary_module`` determines them (``_positions``), or None
+        where they follow from the layer's own settings and the cached tokens."""
+        if position_embeddings is None and position_ids is None and self.rotary_module is None:
+            return None
+        return self._positions(seq_len, position_embeddings, position_ids)
+
+    def _native(self, h16: torch.Tensor, tables: Optional[Tuple] = None) -> bool:
         """Whether ``rfsn_layer_linear`` runs this call's projections: a plain
-        [1, S, hidden] fp16 input nothing watches, weights as it reads them."""
+        [1, S, hidden] fp16 input and rotary tables nothing watches, weights
+        as it reads them."""
         D, qkv = self.hidden_dim, (self.num_heads + 2 * self.num_kv_heads) * self.head_dim
         if (not _unwatched(h16) or h16.dim() != 3 or h16.shape[1] == 0 or int(h16.shape[2]) != D or not h16.is_cuda
-                or h16.device.index != torch.cuda.current_device()):
+                or h16.device.index != torch.cuda.current_device()
+                or not all(_unwatched(t) and t.device == h16.device for t in tables or ())):
             return False
         for name, shape in self._shapes.items():
             w = self._parameters.get(name)
@@ -413,16 +422,17 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         session.left = session.state()
         return out
 
-    def _qkv(self, h16: torch.Tensor, native: bool, position_embeddings, position_ids, q_out=None):
-        """Rotated q and k, and v, [1, S, heads, head_dim] (llama32_adapter.py:570-580)."""
+    def _qkv(self, h16: torch.Tensor, native: bool, tables: Optional[Tuple], q_out=None):
+        """Rotated q and k, and v, [1, S, heads, head_dim] (llama32_adapter.py:570-580); ``tables`` as
+        ``_given_tables`` returns them."""
         S = int(h16.shape[1])
         if not native:
-            return self._project_qkv(h16, *self._positions(S, position_embeddings, position_ids))
+            return self._project_qkv(h16, *(self._positions(S, None, None) if tables is None else tables))
         w = self._parameters
-        if position_embeddings is None and position_ids is None and self.rotary_module is None:
+        if tables is None:
             rope = dict(inv_freq=self._inv_freq(), pos0=self.cache.total_tokens)
         else:
-            cos, sin = self._positions(S, position_embeddings, position_ids)
+            cos, sin = tables
             shape = (S, self.head_dim)
             rope = dict(tables=(cos.expand(shape).contiguous(), sin.expand(shape).contiguous()))
         outs = K.layer_linear(self._rows(h16), [w["q_proj"], w["k_proj"], w["v_proj"]], head_dim=self.head_dim,
@@ -462,7 +472,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         if S == 0:
             return
         h16 = hidden_states.to(self.device, torch.float16)
-        _, k, v = self._qkv(h16, self._native(h16), position_embeddings, position_ids)
+        tables = self._given_tables(S, position_embeddings, position_ids)
+        _, k, v = self._qkv(h16, self._native(h16, tables), tables)
         self.cache.update(k[0], v[0], self.quantizer, disk_dir=self.disk_cache_dir)
 
     def forward(self, hidden_states: torch.Tensor, position_embeddings=None, position_ids=None,
@@ -473,12 +484,12 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
             raise ValueError("The Llama adapter currently supports batch size 1 only")
         S = int(hidden_states.shape[1])
         residual = hidden_states.to(self.device, torch.float16)
-        native = self._native(residual)
+        tables = self._given_tables(S, position_embeddings, position_ids)
+        native = self._native(residual, tables)
         session = None
         if use_cache and native and S == 1 and router is None and context_window is None:
             session = self._session()
-        q, k, v = self._qkv(residual, native, position_embeddings, position_ids,
-                            None if session is None else session.q)
+        q, k, v = self._qkv(residual, native, tables, None if session is None else session.q)
         if session is not None:
             attended = self._session_step(session, k[0], v[0])
         elif use_cache:

@@ -248,3 +248,63 @@ def test_llama_layer_session_follows_its_cache(device, tmp_path):
         layer.prefill_cache(prompt)
     a, b = (H(layer(x, use_cache=True)) for layer in layers)
     assert np.abs(a - b).max() <= 4e-3
+
+
+def _llama(device, tmp_path, **kw):
+    from apple_amd.layer import Llama32DecoderLayerMLX
+
+    cfg = _ext_config(tmp_path)
+    return Llama32DecoderLayerMLX(cfg, intermediate_size=256, device=device, quantizer=_ext_quantizer(cfg, device, 8),
+                                  generator=torch.Generator().manual_seed(4), **kw)
+
+
+def test_llama_layer_watched_tables(device, tmp_path):
+    """Gradients of rotary tables (given, or made by a trainable rotary module) and tables mapped by vmap go through
+    torch's operators; the same tables unwatched agree with them."""
+    from apple_amd.layer import rope_cos_sin
+
+    layer = _llama(device, tmp_path / "a")
+    g = rng(36)
+    x = torch.from_numpy(randn16(g, 1, 6, 512)).to(device)
+    cos, sin = rope_cos_sin(torch.arange(3, 9, device=device), 64)
+    plain = layer(x, position_embeddings=(cos, sin))
+    assert layer._native(x, (cos, sin)) and not plain.requires_grad
+    for i in (0, 1):
+        t = [cos.clone(), sin.clone()]
+        t[i].requires_grad_()
+        out = layer(x, position_embeddings=tuple(t))
+        assert out.requires_grad and (out - plain).abs().max() <= 4e-3
+        out.float().sum().backward()
+        assert t[i].grad is not None and bool(t[i].grad.any())
+        with torch.no_grad():
+            assert torch.equal(layer(x, position_embeddings=tuple(t)), plain)
+    many = torch.func.vmap(lambda c, s: layer(x, position_embeddings=(c, s)))(torch.stack([cos, sin]), torch.stack([sin, cos]))
+    assert (many[0] - plain).abs().max() <= 4e-3
+
+    class Trained(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.shift = torch.nn.Parameter(torch.zeros((), device=device))
+
+        def forward(self, hidden, position_ids):
+            return tuple(t + self.shift for t in rope_cos_sin(position_ids.reshape(-1), 64))
+
+    rot = Trained()
+    layer = _llama(device, tmp_path / "b", rotary_module=rot)
+    out = layer(x)
+    assert out.requires_grad
+    out.float().sum().backward()
+    assert rot.shift.grad is not None and float(rot.shift.grad) != 0.0
+
+
+def test_llama_layer_functional_weights(device, tmp_path):
+    """torch.func.grad and vmap over the layer's weights with a plain input."""
+    layer = _llama(device, tmp_path)
+    x = torch.from_numpy(randn16(rng(37), 1, 5, 512)).to(device)
+    w = layer.down_proj.detach()
+    call = lambda t: torch.func.functional_call(layer, {"down_proj": t}, (x,))
+    grad = torch.func.grad(lambda t: call(t).float().sum())(w)
+    assert grad.shape == w.shape and bool(grad.any())
+    many = torch.func.vmap(call)(torch.stack([w, 2 * w]))
+    plain = layer(x)
+    assert (many[0] - plain).abs().max() <= 4e-3 and not torch.equal(many[0], many[1])
