@@ -27,6 +27,7 @@ from __future__ import annotations
 import itertools
 import math
 import shutil
+import threading
 from pathlib import Path
 from typing import Dict, Optional, Tuple
 
@@ -38,6 +39,8 @@ from .quantization import HybridQuantizerMLX
 from .storage import AsyncHierarchicalRouterMLX, RFSNConfig
 
 MASK_FILL_VALUE = -1e30
+
+_INV_FREQ_LOCK = threading.Lock()  # two calls that miss a layer's kept frequencies make them once
 
 
 def _gelu(x: torch.Tensor) -> torch.Tensor:
@@ -299,6 +302,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         self.rope_scaling = dict(rope_scaling) if rope_scaling else None
         if self.rope_scaling:
             rope_inv_freq(config.head_dim, rope_theta, self.rope_scaling)  # rejects unsupported types now
+        if self.device.type == "cuda":
+            self._inv_freq()
         self.rotary_module = rotary_module
         D, H, Hkv, I = config.hidden_dim, config.num_heads, self.num_kv_heads, intermediate_size
         shapes = {"input_layernorm": (D,), "post_attention_layernorm": (D,), "q_proj": (H * self.head_dim, D),
@@ -384,12 +389,25 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         return x.clone() if x.data_ptr() % 16 else x
 
     def _inv_freq(self) -> torch.Tensor:
-        """``rope_inv_freq`` on the device, rebuilt when the layer's rotary settings change."""
+        """``rope_inv_freq`` on the device, kept for the layer's present rotary settings.  Calls on any stream read
+        it, so its stream is waited for once, where it is made (at construction, for the first settings), and the
+        device before one of other settings is dropped.  Inside a graph capture, where nothing may be waited for
+        and what is made holds nothing before the replay, a missing one is made for the call alone."""
         key = (self.head_dim, self.rope_theta, None if not self.rope_scaling else dict(self.rope_scaling))
-        if getattr(self, "_inv_freq_key", None) != key:
-            self._inv_freq_memo = rope_inv_freq(*key, self.device).contiguous()
-            self._inv_freq_key = key
-        return self._inv_freq_memo
+        kept = self.__dict__.get("_inv_freq_kept")
+        if kept is None or kept[0] != key:
+            with _INV_FREQ_LOCK:
+                kept = self.__dict__.get("_inv_freq_kept")
+                if kept is None or kept[0] != key:
+                    made = (key, rope_inv_freq(*key, self.device).contiguous())
+                    if torch.cuda.is_current_stream_capturing():
+                        return made[1]
+                    if kept is None:
+                        torch.cuda.current_stream(self.device).synchronize()
+                    else:
+                        torch.cuda.synchronize(self.device)
+                    self._inv_freq_kept = kept = made
+        return kept[1]
 
     def _session(self):
         """The decode session of a cached step over the whole hot + warm window
@@ -412,8 +430,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         return s
 
     def __getstate__(self):
-        # the session's prepared launch holds device addresses: a copy of the layer builds its own
-        return {n: v for n, v in self.__dict__.items() if n != "_decode"}
+        # the session's prepared launch and the kept frequencies belong to this layer's device: a copy makes its own
+        return {n: v for n, v in self.__dict__.items() if n not in ("_decode", "_inv_freq_kept")}
 
     def _session_step(self, session, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         session.left = None  # a step that raises leaves a launch to rebuild

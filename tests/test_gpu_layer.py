@@ -308,3 +308,30 @@ def test_llama_layer_functional_weights(device, tmp_path):
     many = torch.func.vmap(call)(torch.stack([w, 2 * w]))
     plain = layer(x)
     assert (many[0] - plain).abs().max() <= 4e-3 and not torch.equal(many[0], many[1])
+
+
+def test_llama_layer_frequencies_on_every_stream(device, tmp_path):
+    """The rotary frequencies that calls on any stream read are complete before the first of them; a graph capture
+    that finds none leaves none behind, and its replays agree with the eager call."""
+    layer = _llama(device, tmp_path)
+    x = torch.from_numpy(randn16(rng(38), 1, 70, 512)).to(device)
+    kept = layer.__dict__["_inv_freq_kept"]
+    with torch.cuda.stream(torch.cuda.Stream(device)):
+        plain = layer(x)
+        assert layer.__dict__["_inv_freq_kept"] is kept  # nothing made on the call's stream
+        torch.cuda.synchronize()
+    del layer._inv_freq_kept
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(x)
+    assert "_inv_freq_kept" not in layer.__dict__
+    eager = layer(x)  # before any replay: reads frequencies of its own
+    torch.cuda.synchronize()
+    assert torch.equal(eager, plain) and "_inv_freq_kept" in layer.__dict__
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, plain) and torch.equal(layer(x), plain)
+    layer.rope_theta = 10000.0
+    assert not torch.equal(layer(x), plain) and layer._inv_freq_kept[0][1] == 10000.0
