@@ -303,7 +303,9 @@ def blockwise_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tenso
     # partials of the splits a launch may choose: enough blocks to fill the
     # chip, so few once there are many query rows
     rows = B * max(1, Hq // max(Hkv, 1))
-    splits_max = max(1, min(1024, -(-T // 256), max(-(-1024 // (B * Hkv)), -(-512 // (Hkv * -(-rows // 256))))))
+    heads = max(Hkv, 1)  # sizes of 0 are the launch's to refuse
+    splits_max = max(1, min(1024, -(-T // 256), max(-(-1024 // max(B * heads, 1)),
+                                                    -(-512 // (heads * max(-(-rows // 256), 1))))))
     wsb = lib.rfsn_attention_workspace_bytes(B, Hq, D, splits_max)
     ws = torch.empty(wsb, dtype=torch.uint8, device=q.device)
     L.call("rfsn_blockwise_attention", q.data_ptr(), B, Hq, D, keys.data_ptr() if T else None,

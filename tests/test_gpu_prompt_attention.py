@@ -104,3 +104,15 @@ def test_hybrid_attention_decodes_once_for_many_queries(device, monkeypatch, fmt
     for out in (got, reg):
         err = np.abs(out.double().cpu().numpy() - want)
         assert np.all(err <= np.abs(want) * 2.0 ** -11 + np.abs(v).max().astype(np.float64) * 2.0 ** -15)
+
+
+@pytest.mark.parametrize("T", [0, 5])
+@pytest.mark.parametrize("B,Hkv", [(0, 2), (3, 0)])
+def test_empty_sizes_are_refused(device, T, B, Hkv):
+    """No queries, or no KV heads: the launch's ValueError, whatever the window."""
+    import torch
+    from apple_amd import kernels as K
+
+    z = lambda *s: torch.zeros(s, dtype=torch.float16, device=device)
+    with pytest.raises(ValueError):
+        K.blockwise_attention(z(B, 2, 64), z(T, Hkv, 64), z(T, Hkv, 64), 0.125, False, None)
