@@ -122,11 +122,17 @@ class RFSNHybridAttentionMLX:
         tables = {}
         use_tables = (tol is not None and not quantizer.subspace and B * Hq <= REF_TABLES_MAX_QUERY_HEADS
                       and T >= K.ref_tables_min_tokens(Hq // key_store.num_heads, B))
-        if K.decode_first(B, Hq, key_store.num_heads, int(q.shape[-1]), T, use_tables):
+        if (B >= K.DECODE_FIRST_QUERIES
+                and K.decode_first(B, Hq, key_store.num_heads, int(q.shape[-1]), T, use_tables,
+                                   quantizer.config.hybrid_window_bytes)):
             # a chunk of a prompt: rebuild each vector once, then attend on the matrix cores
-            out = K.blockwise_attention(q.to(device=dev, dtype=torch.float16), _decode_compressed_tensor(kst, quantizer),
-                                        _decode_compressed_tensor(vst, quantizer), self.scale, causal, pos)
-            return out.to(q.dtype)
+            try:
+                out = K.blockwise_attention(q.to(device=dev, dtype=torch.float16),
+                                            _decode_compressed_tensor(kst, quantizer),
+                                            _decode_compressed_tensor(vst, quantizer), self.scale, causal, pos)
+                return out.to(q.dtype)
+            except torch.OutOfMemoryError:
+                pass  # no room for the decoded window: the kernel below needs none
         if use_tables:
             tables = dict(score_tables=float(tol), table_stats=self._table_stats(quantizer))
         # the tables read a head's codes in whole lines from a head-major

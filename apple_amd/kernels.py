@@ -920,7 +920,11 @@ def ref_tables_min_tokens(group: int, queries: int = 1) -> int:
     return base * (q + 1) // (2 * q)
 
 
-def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, tokens: int, tables: bool) -> bool:
+DECODE_FIRST_QUERIES = 4  # fewest queries for which ``decode_first`` may hold
+
+
+def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, tokens: int, tables: bool,
+                 window_bytes: int = 1 << 30) -> bool:
     """Whether ``queries`` query tokens over ``tokens`` coded ones are faster
     as decode-once-then-attend (``decode_ref`` / ``decode``, then the matrix
     cores' ``blockwise_attention``) than decoded in registers per query.
@@ -933,11 +937,11 @@ def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, token
     whatever the window, decoding 3.3 us per 2^20 coordinates whatever the
     queries: even near queries * q_heads * 2^18 = tokens * kv_heads * D (12,000
     tokens x 32 heads: 120 against 150 us at 4 queries, 211 against 150 at 8).
-    The decoded window is at most 1 GiB for K and V together."""
+    The decoded window takes at most ``window_bytes`` for K and V together."""
     if head_dim not in (64, 128) or kv_heads <= 0 or q_heads % kv_heads or q_heads // kv_heads not in (1, 2, 4, 8):
         return False
     window = tokens * kv_heads * head_dim
-    if queries < 4 or window > 1 << 28:
+    if queries < DECODE_FIRST_QUERIES or 4 * window > window_bytes:
         return False
     if tables:
         return queries * q_heads << 18 >= window

@@ -83,6 +83,10 @@ class RFSNConfig:
     # tolerance recomputes its output on the exact codebook path; None: no
     # guard (the K sparse entries then carry no corrected-coordinate plane)
     score_table_tolerance: Optional[float] = 2e-3
+    # most bytes of fp16 K and V together that RFSNHybridAttentionMLX decodes a
+    # window into for a chunk of queries; larger windows (0: all) keep the
+    # kernel that decodes in registers and needs no such buffer
+    hybrid_window_bytes: int = 1 << 30
 
     def __post_init__(self) -> None:
         expected = self.num_subspaces * self.subspace_dim
@@ -99,6 +103,8 @@ class RFSNConfig:
             raise ValueError("cold_medium must be 'npz' or 'pinned'")
         if self.score_table_tolerance is not None and not self.score_table_tolerance >= 0:
             raise ValueError("score_table_tolerance must be None or >= 0")
+        if self.hybrid_window_bytes < 0:
+            raise ValueError("hybrid_window_bytes must be >= 0")
 
     @property
     def kv_heads(self) -> int:

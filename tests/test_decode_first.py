@@ -1,6 +1,9 @@
 """Which hybrid-attention calls decode their window once (kernels.decode_first)."""
 
+import pytest
+
 from apple_amd.kernels import decode_first
+from apple_amd.storage import RFSNConfig
 
 
 def test_decode_first_lines():
@@ -12,3 +15,8 @@ def test_decode_first_lines():
     assert not decode_first(128, 32, 32, 256, 4096, False)      # no matrix-core kernel of that head_dim
     assert not decode_first(128, 24, 8, 128, 4096, False)       # nor of three query heads per KV head
     assert not decode_first(128, 32, 32, 128, 70_000, False)    # a decoded window over 1 GiB
+    assert not decode_first(128, 32, 32, 128, 4096, False, (1 << 26) - 1)  # or over the caller's limit: 64 MiB
+    assert decode_first(128, 32, 32, 128, 4096, False, 1 << 26)
+    assert not decode_first(128, 32, 32, 128, 4096, False, 0)
+    with pytest.raises(ValueError):
+        RFSNConfig(hybrid_window_bytes=-1)

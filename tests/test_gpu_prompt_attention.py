@@ -6,6 +6,8 @@ rounding (2^-11 of the value) plus fp32 sums of weights kept to 22 bits, so
 2^-11 |out| + 2^-15 max|v| (2^-22 per weight and 2^-24 per product would be
 far below the second term; it covers the exponent of a score of up to 64)."""
 
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -97,8 +99,23 @@ def test_hybrid_attention_decodes_once_for_many_queries(device, monkeypatch, fmt
     assert K.decode_first(B, Hq, Hkv, D, T, False)
     att = A.RFSNHybridAttentionMLX(cfg)
     got = att(q, ks, vs, qz, causal=True, query_positions=pos)
+    # without room for the decoded window, or where the caller declines it, the chunk keeps the kernel in registers
+    decoded = []
+
+    def no_room(store, quantizer):
+        decoded.append(store)
+        raise torch.OutOfMemoryError("no room")
+
+    with monkeypatch.context() as m:
+        m.setattr(A, "_decode_compressed_tensor", no_room)
+        reg = att(q, ks, vs, qz, causal=True, query_positions=pos)
+        assert len(decoded) == 1
+        qz.config = dataclasses.replace(cfg, hybrid_window_bytes=0)
+        declined = att(q, ks, vs, qz, causal=True, query_positions=pos)
+        assert len(decoded) == 1 and torch.equal(declined, reg)
+        qz.config = cfg
     monkeypatch.setattr(K, "decode_first", lambda *a: False)
-    reg = att(q, ks, vs, qz, causal=True, query_positions=pos)
+    assert torch.equal(att(q, ks, vs, qz, causal=True, query_positions=pos), reg)
     k, v = (_decode_compressed_tensor(s, qz).cpu().numpy() for s in (ks, vs))
     want = _ref(q.cpu().numpy(), k, v, D ** -0.5, np.repeat(pos.cpu().numpy()[:, None], Hq, 1))
     for out in (got, reg):
