@@ -305,17 +305,13 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         if self.device.type == "cuda":
             self._inv_freq()
         self.rotary_module = rotary_module
-        D, H, Hkv, I = config.hidden_dim, config.num_heads, self.num_kv_heads, intermediate_size
-        shapes = {"input_layernorm": (D,), "post_attention_layernorm": (D,), "q_proj": (H * self.head_dim, D),
-                  "k_proj": (Hkv * self.head_dim, D), "v_proj": (Hkv * self.head_dim, D),
-                  "o_proj": (D, H * self.head_dim), "gate_proj": (I, D), "up_proj": (I, D), "down_proj": (D, I)}
-        self._shapes = {n: torch.Size(s) for n, s in shapes.items()}
+        shapes = self._shapes = self._weight_shapes(intermediate_size)
         g = generator if generator is not None else torch.Generator().manual_seed(4321 + layer_idx)
         for name in self.WEIGHTS:
             if weights is not None:
                 w = torch.as_tensor(weights[name]).float()
-                if tuple(w.shape) != shapes[name]:
-                    raise ValueError(f"{name}: expected shape {shapes[name]}, got {tuple(w.shape)}")
+                if w.shape != shapes[name]:
+                    raise ValueError(f"{name}: expected shape {tuple(shapes[name])}, got {tuple(w.shape)}")
                 p = torch.nn.Parameter(w.to(self.device), requires_grad=False)
             elif len(shapes[name]) == 1:
                 p = torch.nn.Parameter(torch.ones(shapes[name], device=self.device), requires_grad=False)
@@ -325,6 +321,13 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         self.quantizer = quantizer if quantizer is not None else HybridQuantizerMLX(config, device=self.device)
         self.disk_cache_dir = Path(config.disk_cache_dir) / f"llama_layer_{layer_idx}"
         self.cache = RFSNv10KVCacheMLX(config, layer_idx=layer_idx, device=self.device)
+
+    def _weight_shapes(self, inter: int) -> Dict[str, torch.Size]:
+        D, qd, kvd = self.hidden_dim, self.num_heads * self.head_dim, self.num_kv_heads * self.head_dim
+        shapes = {"input_layernorm": (D,), "post_attention_layernorm": (D,), "q_proj": (qd, D), "k_proj": (kvd, D),
+                  "v_proj": (kvd, D), "o_proj": (D, qd), "gate_proj": (inter, D), "up_proj": (inter, D),
+                  "down_proj": (D, inter)}
+        return {n: torch.Size(s) for n, s in shapes.items()}
 
     @property
     def cache_tokens(self) -> int:
@@ -432,6 +435,11 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
     def __getstate__(self):
         # the session's prepared launch and the kept frequencies belong to this layer's device: a copy makes its own
         return {n: v for n, v in self.__dict__.items() if n not in ("_decode", "_inv_freq_kept")}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if "_shapes" not in self.__dict__:  # a layer saved before it kept its weights' shapes
+            self._shapes = self._weight_shapes(int(self.down_proj.shape[1]))
 
     def _session_step(self, session, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         session.left = None  # a step that raises leaves a launch to rebuild

@@ -335,3 +335,16 @@ def test_llama_layer_frequencies_on_every_stream(device, tmp_path):
         assert torch.equal(out, plain) and torch.equal(layer(x), plain)
     layer.rope_theta = 10000.0
     assert not torch.equal(layer(x), plain) and layer._inv_freq_kept[0][1] == 10000.0
+
+
+def test_llama_layer_saved_without_shapes(device, tmp_path):
+    """A layer pickled before it kept its weights' shapes runs, and as the one it was saved from."""
+    import copy
+
+    layer = _llama(device, tmp_path)
+    state = copy.deepcopy(layer.__getstate__())
+    del state["_shapes"]
+    old = type(layer).__new__(type(layer))
+    old.__setstate__(state)
+    x = torch.from_numpy(randn16(rng(39), 1, 9, 512)).to(device)
+    assert old._shapes == layer._shapes and torch.equal(old(x), layer(x))
