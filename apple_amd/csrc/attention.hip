@@ -308,25 +308,35 @@ static int choose_splits(int64_t T, int64_t blocks_per_split) {
   return (int)s;
 }
 
-extern "C" int rfsn_blockwise_attention(const void* q, int32_t B, int32_t Hq, int32_t D, const void* k, const void* v,
-                                        int64_t T, int32_t Hkv, int64_t stride_t, int64_t stride_h, float scale,
-                                        int32_t causal, const int32_t* qpos, void* out, void* ws, size_t ws_bytes,
-                                        void* stream) {
+// Checks shared by the exact attention entries.
+static int check_exact(const void* q, int32_t B, int32_t Hq, int32_t D, const void* k, const void* v, int64_t T,
+                       int32_t Hkv, int64_t stride_t, int64_t stride_h, const void* out, const void* ws,
+                       size_t ws_bytes) {
   RFSN_REQUIRE(q && out && B > 0 && Hq > 0 && Hkv > 0, "blockwise_attention: bad arguments");
   RFSN_REQUIRE(Hq % Hkv == 0, "blockwise_attention: query heads must be a multiple of KV heads");
   RFSN_REQUIRE(D == 64 || D == 128, "blockwise_attention: head_dim must be 64 or 128");
   RFSN_REQUIRE(T >= 0 && (T == 0 || (k && v)), "blockwise_attention: bad K/V");
   RFSN_REQUIRE(stride_t % 8 == 0 && stride_h % 8 == 0, "blockwise_attention: K/V rows must be 16-byte aligned");
+  RFSN_REQUIRE(ws && ws_bytes >= rfsn_attention_workspace_bytes(B, Hq, D, 1),
+               "blockwise_attention: workspace too small");
+  const int G = Hq / Hkv;
+  if (G != 1 && G != 2 && G != 4 && G != 8)
+    return fail(RFSN_ERR_UNSUPPORTED, "blockwise_attention: Hq/Hkv must be 1, 2, 4 or 8");
+  return RFSN_OK;
+}
+
+extern "C" int rfsn_blockwise_attention(const void* q, int32_t B, int32_t Hq, int32_t D, const void* k, const void* v,
+                                        int64_t T, int32_t Hkv, int64_t stride_t, int64_t stride_h, float scale,
+                                        int32_t causal, const int32_t* qpos, void* out, void* ws, size_t ws_bytes,
+                                        void* stream) {
+  if (int st = check_exact(q, B, Hq, D, k, v, T, Hkv, stride_t, stride_h, out, ws, ws_bytes)) return st;
   const int G = Hq / Hkv;
   hipStream_t s = (hipStream_t)stream;
   const float sl2 = scale * kLog2e;
-  RFSN_REQUIRE(ws && ws_bytes >= rfsn_attention_workspace_bytes(B, Hq, D, 1),
-               "blockwise_attention: workspace too small");
-  if (G != 1 && G != 2 && G != 4 && G != 8)
-    return fail(RFSN_ERR_UNSUPPORTED, "blockwise_attention: Hq/Hkv must be 1, 2, 4 or 8");
+  // a query whose sum of weights is no number yields zeros, from either kernel (launch_merge)
   if (prompt_attention_ok(q, B, Hq, Hkv, D, k, v, T, sl2, out, ws))
-    return launch_prompt_attention(q, B, Hq, Hkv, D, k, v, T, stride_t, stride_h, sl2, causal, qpos, out, ws, ws_bytes,
-                                   s);
+    return launch_prompt_attention(q, B, Hq, Hkv, D, k, v, T, stride_t, stride_h, sl2, causal, qpos, 0.f, out, ws,
+                                   ws_bytes, s);
   int splits = T > 0 ? choose_splits(T, (int64_t)B * Hkv) : 1;
   if (ws_bytes < rfsn_attention_workspace_bytes(B, Hq, D, splits)) splits = 1;
   const int64_t tps = T > 0 ? ceil_div(ceil_div(T, splits), 64) * 64 : 64;
@@ -341,22 +351,33 @@ extern "C" int rfsn_blockwise_attention(const void* q, int32_t B, int32_t Hq, in
       case 1: RFSN_EXACT(64, 1); break;
       case 2: RFSN_EXACT(64, 2); break;
       case 4: RFSN_EXACT(64, 4); break;
-      case 8: RFSN_EXACT(64, 8); break;
-      default: return fail(RFSN_ERR_UNSUPPORTED, "blockwise_attention: Hq/Hkv must be 1, 2, 4 or 8");
+      default: RFSN_EXACT(64, 8); break;
     }
   } else {
     switch (G) {
       case 1: RFSN_EXACT(128, 1); break;
       case 2: RFSN_EXACT(128, 2); break;
       case 4: RFSN_EXACT(128, 4); break;
-      case 8: RFSN_EXACT(128, 8); break;
-      default: return fail(RFSN_ERR_UNSUPPORTED, "blockwise_attention: Hq/Hkv must be 1, 2, 4 or 8");
+      default: RFSN_EXACT(128, 8); break;
     }
   }
 #undef RFSN_EXACT
   int st = check_launch("blockwise_attention");
   if (st) return st;
   return launch_merge((const float*)ws, (int64_t)B * Hq, splits, D, out, s);
+}
+
+extern "C" int rfsn_dense_attention(const void* q, int32_t B, int32_t Hq, int32_t D, const void* k, const void* v,
+                                    int64_t T, int32_t Hkv, int64_t stride_t, int64_t stride_h, float scale,
+                                    int32_t causal, const int32_t* qpos, void* out, void* ws, size_t ws_bytes,
+                                    void* stream) {
+  if (int st = check_exact(q, B, Hq, D, k, v, T, Hkv, stride_t, stride_h, out, ws, ws_bytes)) return st;
+  const float sl2 = scale * kLog2e;
+  if (!prompt_attention_ok(q, B, Hq, Hkv, D, k, v, T, sl2, out, ws))
+    return fail(RFSN_ERR_UNSUPPORTED,
+                "dense_attention: needs 4 query rows per KV head, a positive scale and 16-byte aligned buffers");
+  return launch_prompt_attention(q, B, Hq, Hkv, D, k, v, T, stride_t, stride_h, sl2, causal, qpos, __builtin_nanf(""),
+                                 out, ws, ws_bytes, (hipStream_t)stream);
 }
 
 extern "C" int rfsn_pack_codes(const uint8_t* src, int64_t src_head_stride, int64_t T, int32_t M, int32_t heads,

@@ -14,8 +14,14 @@
 //                  slot (half hf, j) of step st is token 16 st + 8 (j >> 2) +
 //                  4 hf + (j & 3), and ds_read_b64_tr_b16 reads V^T in that
 //                  order from row-major V, so neither P nor V changes lanes.
-// P keeps 22 bits and more, p * 2^8 as fp16 hi + fp16 lo (two MFMAs; V is
-// exact); everything accumulates in fp32, and the row sum adds the unsplit p.
+// P is kept to 2^-23 of itself (exp2's own error), p * 2^8 as fp16 hi + fp16 lo
+// (two MFMAs; V is exact); everything accumulates in fp32, and the row sum adds
+// the unsplit p.  Before its fp16 rounding a result is off by 2.5e-7 to 5.8e-7
+// (2-norm against float64, 64 to 1,000 queries, 500 to 8,192 tokens, scores of
+// deviation 1 to 16); attention.hip's fp32 products of fp32 weights are off by
+// 3.2e-7 to 1.6e-6 on the same inputs.
+// Infinities in V: hi * V and lo * V cancel or meet 0 where p * V is infinite, so
+// a block that finds a NaN in its sums takes its rows again in fp32 (careful_row).
 // The maximum is moved only when a lane's sum of p says that it must be, which
 // takes the max scan and its cross-lane step out of most tiles.
 //
@@ -58,12 +64,55 @@ __device__ __forceinline__ half8 join(const half2v* p) {
   return half8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
 }
 
+// One row over the tokens t0 .. lim by one wave, as attention.hip's kernel takes it:
+// lane = token for scores, lane = coordinate for P V, weights and products in fp32.
+// NaN and infinite values meet the weights of the tokens the row may read, and no
+// others.
+template <int D>
+__device__ __forceinline__ void careful_row(const uint16_t* __restrict__ q, const uint16_t* __restrict__ K,
+                                            const uint16_t* __restrict__ V, int64_t stride_t, float scale_log2, int t0,
+                                            int lim, int lane, float& m, float& l, float (&acc)[D / 64]) {
+  m = -__builtin_inff();
+  l = 0.f;
+#pragma unroll
+  for (int e = 0; e < D / 64; ++e) acc[e] = 0.f;
+#pragma unroll 1
+  for (int base = t0; base <= lim; base += 64) {
+    const bool allowed = base + lane <= lim;
+    const half8* k = reinterpret_cast<const half8*>(K + (int64_t)min(base + lane, lim) * stride_t);
+    float s = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < D / 8; ++c) {
+      const half8 kv = k[c], qv = reinterpret_cast<const half8*>(q)[c];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s = fmaf((float)qv[e] * scale_log2, (float)kv[e], s);
+    }
+    if (!allowed) s = -__builtin_inff();
+    const float mn = fmaxf(m, wave_max(s));
+    const float p = mn > -__builtin_inff() ? exp2f(s - mn) : s != s ? s : 0.f;  // a NaN score is no maximum
+    const float corr = m > -__builtin_inff() ? exp2f(m - mn) : (mn > -__builtin_inff() ? 0.f : 1.f);
+    l = l * corr + wave_sum(p);
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < D / 64; ++e) acc[e] *= corr;
+    const int count = min(64, lim - base + 1);
+#pragma unroll 1
+    for (int t = 0; t < count; ++t) {
+      const float pt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), t));
+      const uint16_t* v = V + (int64_t)(base + t) * stride_t + lane * (D / 64);
+#pragma unroll
+      for (int e = 0; e < D / 64; ++e) acc[e] = fmaf(pt, h2f(v[e]), acc[e]);
+    }
+  }
+}
+
 template <int D, int WR, int WT, int MW>
 __global__ void __launch_bounds__(WR * WT * 64, MW)
 prompt_attn_kernel(const uint16_t* __restrict__ q, int B, int Hq, int G, const uint16_t* __restrict__ K,
                    const uint16_t* __restrict__ V, int T, int64_t stride_t, int64_t stride_h, float scale_log2,
                    int causal, const int32_t* __restrict__ qpos, int row_tiles, int tokens_per_split, int splits,
-                   uint16_t* __restrict__ out, float* __restrict__ part_ml, float* __restrict__ part_acc) {
+                   float bad, uint16_t* __restrict__ out, float* __restrict__ part_ml,
+                   float* __restrict__ part_acc) {
   constexpr int kThreads = WR * 64;                         // threads of a token group
   constexpr int kChunks = D / 8;                            // 16-byte chunks of a row
   constexpr int kLoads = kTile * kChunks / kThreads;        // chunks a thread stages per tile and tensor
@@ -240,6 +289,39 @@ prompt_attn_kernel(const uint16_t* __restrict__ q, int B, int Hq, int G, const u
     __syncthreads();
   }
 
+  bool nan = false;
+#pragma unroll
+  for (int d = 0; d < kDT; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) nan = nan || o[d][i] != o[d][i];
+  nan = __any(nan);
+  if (lane == 0) s_hi[wave] = nan;  // its bounds were read before the barriers above
+  __syncthreads();
+  int any = s_hi[0];
+#pragma unroll
+  for (int w = 1; w < WR * WT; ++w) any |= s_hi[w];
+  if (any) {  // block-uniform: the block's rows again, a wave per row
+    for (int r = wave; r < WR * 32; r += WR * WT) {
+      const int row2 = rt * (WR * 32) + r;
+      if (row2 >= rows) break;
+      const int64_t qr = (int64_t)(row2 / G) * Hq + (int64_t)h * G + row2 % G;
+      int last = min(T, t1) - 1;
+      if (causal && qpos) last = min(last, qpos[qr]);
+      float m, lr, acc[D / 64];
+      careful_row<D>(q + qr * D, Kh, Vh, stride_t, scale_log2, t0, last, lane, m, lr, acc);
+      if (splits > 1) {
+        if (lane == 0) part_ml[2 * (qr * splits + split)] = m, part_ml[2 * (qr * splits + split) + 1] = lr;
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e) part_acc[(qr * splits + split) * D + lane * (D / 64) + e] = acc[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e)
+          out[qr * D + lane * (D / 64) + e] = f2h(lr > 0.f ? acc[e] / lr : lr == 0.f ? 0.f : bad);
+      }
+    }
+    return;
+  }
+
   float l = l_run + __shfl_xor(l_run, 32, 64);
   if constexpr (WT > 1) {
     // groups 1.. hand their (m, l, O) to group 0 through LDS, one at a time
@@ -274,7 +356,7 @@ prompt_attn_kernel(const uint16_t* __restrict__ q, int B, int Hq, int G, const u
   }
   if (row >= rows) return;
   if (splits == 1) {
-    const float inv = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : l);  // nothing allowed: zeros; a NaN sum stays NaN
+    const float inv = l > 0.f ? 1.f / l : 0.f;  // nothing allowed: zeros (a NaN sum has NaN products, handled above)
 #pragma unroll
     for (int d = 0; d < kDT; ++d)
 #pragma unroll
@@ -305,7 +387,7 @@ prompt_attn_kernel(const uint16_t* __restrict__ q, int B, int Hq, int G, const u
 template <int D>
 __global__ void __launch_bounds__(256)
 prompt_merge_kernel(const float* __restrict__ ml, const float* __restrict__ acc, int64_t rows, int splits,
-                    uint16_t* __restrict__ out) {
+                    float bad, uint16_t* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t r = i / (D / 4);
   const int c = (int)(i % (D / 4)) * 4;
@@ -323,14 +405,18 @@ prompt_merge_kernel(const float* __restrict__ ml, const float* __restrict__ acc,
     const float4 v = *reinterpret_cast<const float4*>(acc + (r * splits + s) * D + c);
     a.x += w * v.x, a.y += w * v.y, a.z += w * v.z, a.w += w * v.w;
   }
-  const float inv = l > 0.f ? 1.f / l : (l == 0.f ? 0.f : l);
+  const float inv = 1.f / l;
   half4 o = {(f16)(a.x * inv), (f16)(a.y * inv), (f16)(a.z * inv), (f16)(a.w * inv)};
+  if (!(l > 0.f)) {  // nothing allowed: zeros; a sum that is no number: bad
+    const f16 none = (f16)(l == 0.f ? 0.f : bad);
+    o = half4{none, none, none, none};
+  }
   *reinterpret_cast<half4*>(out + r * D + c) = o;
 }
 
 template <int D, int WR, int WT, int MW>
 int launch(const void* q, int B, int Hq, int G, const void* k, const void* v, int T, int Hkv, int64_t stride_t,
-           int64_t stride_h, float sl2, int causal, const int32_t* qpos, void* out, void* ws, int splits,
+           int64_t stride_h, float sl2, int causal, const int32_t* qpos, float bad, void* out, void* ws, int splits,
            hipStream_t s) {
   const int row_tiles = (int)ceil_div((int64_t)B * G, WR * 32);
   const int tps = (int)(ceil_div(ceil_div(T, splits), kTile) * kTile);
@@ -339,12 +425,12 @@ int launch(const void* q, int B, int Hq, int G, const void* k, const void* v, in
   float* acc = (float*)ws;
   hipLaunchKernelGGL((prompt_attn_kernel<D, WR, WT, MW>), dim3((unsigned)Hkv, (unsigned)row_tiles, (unsigned)splits),
                      dim3(WR * WT * 64), 0, s, (const uint16_t*)q, B, Hq, G, (const uint16_t*)k, (const uint16_t*)v, T,
-                     stride_t, stride_h, sl2, causal, qpos, row_tiles, tps, splits, (uint16_t*)out, acc + slots * D,
-                     acc);
+                     stride_t, stride_h, sl2, causal, qpos, row_tiles, tps, splits, bad, (uint16_t*)out,
+                     acc + slots * D, acc);
   if (splits > 1) {
     const int64_t rows = (int64_t)B * Hq;
     hipLaunchKernelGGL(prompt_merge_kernel<D>, dim3((unsigned)ceil_div(rows * (D / 4), 256)), dim3(256), 0, s,
-                       acc + slots * D, acc, rows, splits, (uint16_t*)out);
+                       acc + slots * D, acc, rows, splits, bad, (uint16_t*)out);
   }
   return check_launch("prompt_attention");
 }
@@ -363,8 +449,8 @@ bool prompt_attention_ok(const void* q, int64_t B, int Hq, int Hkv, int D, const
 }
 
 int launch_prompt_attention(const void* q, int B, int Hq, int Hkv, int D, const void* k, const void* v, int64_t T,
-                            int64_t stride_t, int64_t stride_h, float sl2, int causal, const int32_t* qpos, void* out,
-                            void* ws, size_t ws_bytes, hipStream_t s) {
+                            int64_t stride_t, int64_t stride_h, float sl2, int causal, const int32_t* qpos, float bad,
+                            void* out, void* ws, size_t ws_bytes, hipStream_t s) {
   const int G = Hq / Hkv;
   const int64_t rows = (int64_t)B * G;
   // Rows per block: 64 (two token groups share them) fill the chip soonest and waste
@@ -383,7 +469,7 @@ int launch_prompt_attention(const void* q, int B, int Hq, int Hkv, int D, const 
   if (splits > 64) splits = 64;
   if (splits < 1) splits = 1;
 #define RFSN_PROMPT(DD, WR, WT, MW)                                                                                    \
-  return launch<DD, WR, WT, MW>(q, B, Hq, G, k, v, (int)T, Hkv, stride_t, stride_h, sl2, causal, qpos, out, ws,        \
+  return launch<DD, WR, WT, MW>(q, B, Hq, G, k, v, (int)T, Hkv, stride_t, stride_h, sl2, causal, qpos, bad, out, ws,   \
                                 (int)splits, s)
   if (D == 64) {
     if (wr == 8) RFSN_PROMPT(64, 8, 1, 4);

@@ -11,10 +11,11 @@ int launch_merge(const float* partial, int64_t bh, int splits, int D, void* out,
 // Whether it serves a call (shape, finite positive scale, 16-byte aligned buffers).
 bool prompt_attention_ok(const void* q, int64_t B, int Hq, int Hkv, int D, const void* k, const void* v, int64_t T,
                          float scale_log2, const void* out, const void* ws);
-// The call; split partials go to ws, as many as fit its ws_bytes (none with one split).
+// The call; split partials go to ws, as many as fit its ws_bytes (none with one
+// split).  bad: the output of a query whose sum of weights is no number.
 int launch_prompt_attention(const void* q, int B, int Hq, int Hkv, int D, const void* k, const void* v, int64_t T,
                             int64_t stride_t, int64_t stride_h, float scale_log2, int causal, const int32_t* qpos,
-                            void* out, void* ws, size_t ws_bytes, hipStream_t s);
+                            float bad, void* out, void* ws, size_t ws_bytes, hipStream_t s);
 
 // ---- score tables of rfsn_ref_attention (ref_tables.hip) ----
 // Codebook entries of the tables: M PQ sections of C entries, then L gated

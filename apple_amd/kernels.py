@@ -285,8 +285,10 @@ def _qpos(qpos: torch.Tensor, B: int, Hq: int, device) -> torch.Tensor:
 
 
 def blockwise_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scale: float,
-                        causal: bool, qpos: Optional[torch.Tensor]) -> torch.Tensor:
-    """Exact attention of q [B, Hq, D] over keys/values [T, Hkv, D] (strided rows)."""
+                        causal: bool, qpos: Optional[torch.Tensor], *, dense: bool = False) -> torch.Tensor:
+    """Exact attention of q [B, Hq, D] over keys/values [T, Hkv, D] (strided rows).
+    ``dense``: a query whose scores hold a NaN yields NaN, as a dense softmax,
+    and not zeros (``dense_attention_ok`` calls only)."""
     _dev(q, "blockwise_attention")
     q = _contig(q)
     B, Hq, D = q.shape
@@ -308,10 +310,16 @@ def blockwise_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tenso
                                                     -(-512 // (heads * max(-(-rows // 256), 1))))))
     wsb = lib.rfsn_attention_workspace_bytes(B, Hq, D, splits_max)
     ws = torch.empty(wsb, dtype=torch.uint8, device=q.device)
-    L.call("rfsn_blockwise_attention", q.data_ptr(), B, Hq, D, keys.data_ptr() if T else None,
-           values.data_ptr() if T else None, T, Hkv, keys.stride(0), keys.stride(1), float(scale), int(causal),
+    L.call("rfsn_dense_attention" if dense else "rfsn_blockwise_attention", q.data_ptr(), B, Hq, D,
+           keys.data_ptr() if T else None, values.data_ptr() if T else None, T, Hkv, keys.stride(0), keys.stride(1), float(scale), int(causal),
            L.ptr(qp), out.data_ptr(), ws.data_ptr(), wsb, _stream(q))
     return out
+
+
+def dense_attention_ok(queries: int, q_heads: int, kv_heads: int, head_dim: int, scale: float) -> bool:
+    """Whether ``blockwise_attention(dense=True)`` serves buffers of its own making of this shape."""
+    return (head_dim in (64, 128) and kv_heads > 0 and q_heads % kv_heads == 0 and q_heads // kv_heads in (1, 2, 4, 8)
+            and queries * (q_heads // kv_heads) >= 4 and 0.0 < scale < 1e30)
 
 
 def pack_codes(src: torch.Tensor, dst: torch.Tensor, t_base: int) -> None:

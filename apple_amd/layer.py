@@ -526,9 +526,9 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
             attended = self.cache.attention_forward(
                 q[:, 0], causal=True, router=router, current_position=pos, context_window=context_window,
             ).reshape(1, 1, self.num_heads, self.head_dim)
-        elif native and S and self.head_dim in (64, 128) and self.num_key_value_groups in (1, 2, 4, 8):
+        elif native and K.dense_attention_ok(S, self.num_heads, self.num_kv_heads, self.head_dim, self.scale):
             own = torch.arange(S, dtype=torch.int32, device=self.device)[:, None].expand(S, self.num_heads)
-            attended = K.blockwise_attention(q[0], k[0], v[0], self.scale, True, own)
+            attended = K.blockwise_attention(q[0], k[0], v[0], self.scale, True, own, dense=True)
         else:
             g = self.num_key_value_groups
             attended = _dense_exact_attention(q, _repeat_kv(k, g), _repeat_kv(v, g), self.scale, causal=True)

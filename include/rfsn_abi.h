@@ -193,13 +193,26 @@ int rfsn_decode_ref(const uint8_t* pq_codes_dev, int64_t n, int32_t D, int32_t M
  * Hq % Hkv == 0 (query head h reads KV head h / (Hq/Hkv)),
  * qpos_dev [B][Hq] int32 or NULL (= every query at T-1), causal masks
  * positions > qpos; out [B][Hq][D] fp16 = q.dtype.  Any block size gives the
- * same result up to fp32 rounding. */
+ * same result up to fp32 rounding.  A query without an allowed position, and
+ * one whose sum of weights is no number (a NaN in its scores), yields zeros.
+ * Infinite and NaN values at positions a query may read reach its output; with
+ * fewer than 4 query rows per KV head (B * Hq / Hkv) those at masked positions
+ * may make it NaN too. */
 size_t rfsn_attention_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t splits);
 int rfsn_blockwise_attention(const void* q_dev, int32_t B, int32_t Hq, int32_t D,
                              const void* k_dev, const void* v_dev, int64_t T, int32_t Hkv,
                              int64_t stride_t, int64_t stride_h, float scale, int32_t causal,
                              const int32_t* qpos_dev, void* out_dev,
                              void* workspace_dev, size_t workspace_bytes, void* stream);
+/* The same for a prompt's dense causal attention (attention.py:108-134), whose
+ * softmax carries a NaN on: a query whose sum of weights is no number yields
+ * NaN.  Serves at least 4 query rows per KV head (B * Hq / Hkv), a positive
+ * scale and 16-byte aligned buffers; refuses other calls. */
+int rfsn_dense_attention(const void* q_dev, int32_t B, int32_t Hq, int32_t D,
+                         const void* k_dev, const void* v_dev, int64_t T, int32_t Hkv,
+                         int64_t stride_t, int64_t stride_h, float scale, int32_t causal,
+                         const int32_t* qpos_dev, void* out_dev,
+                         void* workspace_dev, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------- decoder layer
  * y = x W^T of the decoder layer's projections (llama32_adapter.py:555-587):

@@ -133,3 +133,76 @@ def test_empty_sizes_are_refused(device, T, B, Hkv):
     z = lambda *s: torch.zeros(s, dtype=torch.float16, device=device)
     with pytest.raises(ValueError):
         K.blockwise_attention(z(B, 2, 64), z(T, Hkv, 64), z(T, Hkv, 64), 0.125, False, None)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,D", [(4, 2, 2, 1, 64), (5, 8, 4, 63, 64), (33, 4, 2, 65, 128), (65, 2, 2, 1537, 128),
+                                          (150, 4, 2, 1600, 64), (600, 4, 2, 6200, 64), (7, 8, 1, 5000, 64)])
+def test_infinite_values(device, B, Hq, Hkv, T, D):
+    """Infinite values meet every weight as p * V does: infinities where one sign is seen, NaN where both are, and the
+    other coordinates as without them; from many query rows as from one (the scalar kernel)."""
+    import torch
+    from apple_amd import kernels as K
+
+    g = np.random.default_rng(T)
+    q, k, v = (g.standard_normal(s, dtype=np.float32).astype(np.float16)
+               for s in ((B, Hq, D), (T, Hkv, D), (T, Hkv, D)))
+    want = _ref(q, k, v, D ** -0.5, None)
+    v[T - 1, :, 1] = np.inf                              # the last token, which the tiles' ends repeat
+    v[T // 2, :, 7] = v[T // 3, :, 7] = -np.inf
+    v[0, :, D - 1], v[T - 1, :, D - 1] = np.inf, -np.inf
+    v[T // 2, 0, 9] = np.nan
+    want[:, :, 1], want[:, :, 7] = np.inf, -np.inf
+    want[:, :, D - 1] = np.nan if T > 1 else -np.inf
+    want[:, :Hq // Hkv, 9] = np.nan
+    dev = lambda a: torch.from_numpy(a).to(device)
+    tol = np.where(np.isfinite(want), np.abs(want), 0) * 2.0 ** -11 + 6 * 2.0 ** -15
+    runs = [K.blockwise_attention(dev(q), dev(k), dev(v), D ** -0.5, False, None, dense=d) for d in (False, True)]
+    if Hq == Hkv:  # one query row per KV head: the scalar kernel
+        runs.append(torch.cat([K.blockwise_attention(dev(q[i:i + 1]), dev(k), dev(v), D ** -0.5, False, None)
+                               for i in range(B)]))
+    for got in runs:
+        got = got.double().cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        same = np.isfinite(want)
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        assert np.all(np.abs(got[same] - want[same]) <= tol[same])
+    # a causal chunk: every row as the values it may read make it, and no others
+    if B * Hq // Hkv >= 4:
+        pos = g.integers(-1, T, (B, Hq)).astype(np.int32)
+        got = K.blockwise_attention(dev(q), dev(k), dev(v), D ** -0.5, True, dev(pos)).double().cpu().numpy()
+        fin = np.where(np.isfinite(v), v, np.float16(0))
+        want = _ref(q, k, fin, D ** -0.5, pos)
+        seen = (np.arange(T)[None, None] <= pos[..., None])[..., None]           # [B, Hq, T, 1]
+        vh = np.repeat(v, Hq // Hkv, 1).transpose(1, 0, 2)[None]                   # [1, Hq, T, D]
+        up, down, nan = ((seen & f(vh)).any(2) for f in (np.isposinf, np.isneginf, np.isnan))
+        want[up], want[down], want[nan | (up & down)] = np.inf, -np.inf, np.nan
+        same = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        assert np.all(np.abs(got[same] - want[same]) <= np.abs(want[same]) * 2.0 ** -11 + 6 * 2.0 ** -15)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,D", [(1, 2, 2, 70, 64), (6, 2, 2, 70, 64), (40, 4, 2, 1500, 128)])
+def test_scores_that_are_no_numbers(device, B, Hq, Hkv, T, D):
+    """A NaN in a query, or in a key it may see: zeros from blockwise attention, whatever the number of query rows
+    (one is the scalar kernel's), and NaN from dense attention; keys past a query's position change nothing."""
+    import torch
+    from apple_amd import kernels as K
+
+    g = np.random.default_rng(T)
+    q, k, v = (g.standard_normal(s, dtype=np.float32).astype(np.float16)
+               for s in ((B, Hq, D), (T, Hkv, D), (T, Hkv, D)))
+    pos = np.repeat((np.arange(B) + T - B)[:, None], Hq, 1).astype(np.int32)
+    want = _ref(q, k, v, D ** -0.5, pos)
+    k[T - 1, 0, 3] = np.nan                              # the last query's own key
+    q[B // 2, -1, 5] = np.nan
+    bad = np.zeros((B, Hq), bool)
+    bad[B - 1, :Hq // Hkv] = bad[B // 2, -1] = True
+    dev = lambda a: torch.from_numpy(a).to(device)
+    for dense in (False, True) if B * Hq // Hkv >= 4 else (False,):
+        got = K.blockwise_attention(dev(q), dev(k), dev(v), D ** -0.5, True, dev(pos), dense=dense)
+        got = got.double().cpu().numpy()
+        assert (np.isnan(got[bad]).all() if dense else not got[bad].any())
+        assert np.all(np.abs(got - want)[~bad] <= np.abs(want[~bad]) * 2.0 ** -11 + 5 * 2.0 ** -15)
+    if B == 1:
+        with pytest.raises(Exception, match="dense_attention"):
+            K.blockwise_attention(dev(q), dev(k), dev(v), D ** -0.5, True, dev(pos), dense=True)
