@@ -138,6 +138,11 @@ __global__ void __launch_bounds__(256, 4) linear_row_kernel(const rfsn_linear_pa
   float a = 0.f, b = 0.f;
   for (int base = k0; base < k1; base += kRowSlice) {
     if (base != k0) fetch(base);
+    if (base + kRowSlice > k1) {  // past the slice's end: weights that are not its own, infinite perhaps
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (base + u * 256 + lane * 4 >= k1) wa[u] = wb[u] = (float4v)0.f;
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = base + u * 256 + lane * 4;

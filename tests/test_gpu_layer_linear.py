@@ -112,6 +112,34 @@ def test_weights_outside_the_first_scale(device, rows):
     assert np.all(np.delete(ok, 9, 1))
 
 
+@pytest.mark.parametrize("k", [64, 192, 320, 2048, 2112, 8192, 8256, 32768])
+def test_one_row_infinite_weights(device, k):
+    """Infinite weights anywhere in a row, of one row of x: at the ends of k, of its 2,048-wide rounds and of the
+    quarters that waves share from 8,192 on (the loads past a wave's share are not its own), and the widest k."""
+    from apple_amd import kernels as K
+
+    g, x, w = _data(1, k, 128, k)
+    x = np.where(x == 0, np.float16(1), x)
+    quarter = k // 4 if k >= 8192 else k
+    spots = sorted({0, k - 1, k - 4, k // 2, min(2047, k - 1), min(2048, k - 1), quarter - 1, quarter % k, 2 * quarter % k})
+    m = w[0].copy()
+    for i, c in enumerate(spots):
+        m[3 * i, c] = np.inf if i % 2 else -np.inf
+    res = np.zeros((1, 128), np.float16)
+    x64 = x.astype(np.float64)
+    want = x64 @ w[0].T.astype(np.float64)
+    mag = np.abs(x64) @ np.abs(w[0].T.astype(np.float64))
+    for i, c in enumerate(spots):
+        want[0, 3 * i] = np.inf * m[3 * i, c] * float(x[0, c])
+    for o in (K.layer_linear(_t(x, device), [_t(m, device)])[0],
+              K.layer_linear(_t(x, device), [_t(m, device)], K.LINEAR_RESIDUAL, residual=_t(res, device))[0]):
+        o = o.double().cpu().numpy()
+        assert np.array_equal(np.isinf(o), np.isinf(want)) and not np.isnan(o).any()
+        f = np.isfinite(want)
+        assert np.array_equal(o[~f], np.sign(want[~f]) * np.inf)
+        assert np.all(np.abs(o[f] - want[f]) <= np.abs(want[f]) * 2.0 ** -11 + mag[f] * 2.0 ** -20 + 2.0 ** -24)
+
+
 def test_refusals(device):
     import torch
     from apple_amd import kernels as K
