@@ -6,12 +6,18 @@
 //  - one row (a decode step): linear_row_kernel, fp32 FMAs, one pass over the
 //    weights;
 //  - more rows: the weights are split on their way to the matrix cores, w =
-//    (hi + lo) / 2^12 with hi, lo fp16 (24 bits less one for |w| in [2^-10,
-//    16), 2^-37 absolute below), and x is exact, so x W^T = MFMA(x, hi) +
-//    MFMA(x, lo) in one fp32 accumulator.  A block whose weights leave fp16's
-//    range at that scale sees it in its own maximum and repeats its work at
-//    scales that fit.  (An infinite x, which fp32 sums would carry as an
-//    infinity, may come out as NaN: its products with hi and lo cancel.)
+//    (hi + lo) / scale with hi, lo fp16, and x is exact, so x W^T = MFMA(x, hi)
+//    + MFMA(x, lo) in one fp32 accumulator.  At the scale of 2^12 a weight keeps
+//    its value to 2^-23 of itself or 2^-37, whichever is more.  A block that
+//    holds a row whose largest weight is past fp16's range there, or below
+//    2^-12, where 2^-37 is no longer little, repeats its work with each row at a
+//    scale of its own: 2^-23 of the weight or 2^-39 of the row's largest.
+//    Measured against float64 as the share of fp16 results that are not the
+//    nearest: 0.12 to 0.35 % (8 to 1,024 rows, k 2,048 and 8,192), torch's fp32
+//    products 0.33 to 0.69 % on the same inputs.
+//    An infinite x times lo would cancel or meet 0, so a block that finds a sum
+//    that is not finite repeats its work too, with infinities kept from the lo product and
+//    hi kept from 0: x W^T is then infinite or NaN as fp32 sums of x w are.
 //
 // The Llama-3.2-1B layer's seven matrices (243 MB of fp32), torch's fp32 products
 // against this file, without the elementwise kernels around the former:
@@ -31,6 +37,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint16_t ushort8 __attribute__((ext_vector_type(8)));
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 constexpr int kModePlain = 0, kModeSwiglu = 1, kModeResidual = 2;
@@ -240,22 +247,18 @@ __global__ void __launch_bounds__(256) rope_rows_kernel(const rfsn_linear_params
   }
 }
 
-// Scale of the weights: 2^12 for every row at first; a block with a weight that
-// leaves fp16's range there (its maximum says so) finds each row's maximum and
-// repeats its work with the largest power of two per row that keeps it below 2^15
+// Scale of the weights: 2^12 for every row at first; where a row's largest weight
+// does not suit that (scale_ok), the largest power of two that keeps it below 2^15
 // (an infinite weight counts as the largest float, and stays infinite).
 constexpr float kScale = 4096.f;
-__device__ __forceinline__ bool scale_ok(float wmax) { return wmax * kScale < 65504.f; }
+__device__ __forceinline__ bool scale_ok(float wmax) {
+  return wmax == 0.f || (wmax >= 0x1p-12f && wmax * kScale < 65504.f);
+}
 __device__ __forceinline__ float scale_for(float wmax) {
   if (scale_ok(wmax)) return kScale;
   int e = 128;
   if (wmax < __builtin_inff()) frexpf(wmax, &e);  // wmax < 2^e
-  return ldexpf(1.f, 15 - e);
-}
-__device__ __forceinline__ float max8(float m, const float4v& a, const float4v& b) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(a[e]), fabsf(b[e])));
-  return m;
+  return ldexpf(1.f, min(15 - e, 100));
 }
 
 // eight consecutive weights as hi and lo halves of w * scale; their maximum folded into wmax
@@ -265,9 +268,13 @@ __device__ __forceinline__ void split8(const float4v& a, const float4v& b, float
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
     const float w0 = e < 4 ? a[e] : b[e - 4], w1 = e < 4 ? a[e + 1] : b[e - 3];
-    wmax = fmaxf(fmaxf(wmax, fabsf(w0)), fabsf(w1));
+    if (!CAREFUL) wmax = fmaxf(fmaxf(wmax, fabsf(w0)), fabsf(w1));
     const float2v s = {w0 * scale, w1 * scale};
-    const half2v h = __builtin_convertvector(s, half2v);
+    half2v h = __builtin_convertvector(s, half2v);
+    if (CAREFUL) {  // hi is 0 for a weight of 0 alone: an infinite x has to meet the others' sign
+      if (h[0] == (f16)0.f && w0 != 0.f) h[0] = (f16)copysignf(0x1p-24f, w0);
+      if (h[1] == (f16)0.f && w1 != 0.f) h[1] = (f16)copysignf(0x1p-24f, w1);
+    }
     float2v r = {fmaf(minus1, (float)h[0], s[0]), fmaf(minus1, (float)h[1], s[1])};
     if (CAREFUL) {  // an infinite weight stays infinite
       if (!(fabsf(s[0]) < __builtin_inff())) r[0] = 0.f;
@@ -279,14 +286,12 @@ __device__ __forceinline__ void split8(const float4v& a, const float4v& b, float
   }
 }
 
-__device__ __forceinline__ float block_max(float v, float* red, int waves) {
-  v = wave_max(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float m = red[0];
-  for (int w = 1; w < waves; ++w) m = fmaxf(m, red[w]);
-  return m;
+// x with 0 for its infinities and NaN: what lo is multiplied by where some may be
+__device__ __forceinline__ half8 finite8(half8 x) {
+  const ushort8 b = __builtin_bit_cast(ushort8, x);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (b[e] & 0x7C00) == 0x7C00 ? (f16)0.f : x[e];
+  return x;
 }
 
 // Output rows r .. r + 3 (of one matrix: sizes are multiples of 4) at row s of x,
@@ -347,7 +352,7 @@ __global__ void __launch_bounds__(W * 64)
 linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, int rows) {
   constexpr int AN = MODE == kModeSwiglu ? 2 : 1;
   __shared__ float4v sums[W][AN * CT][64];
-  __shared__ float red[W];
+  __shared__ int again;
   __shared__ int row_max[AN * 16];
   __shared__ float row_inv[AN * 16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -364,13 +369,16 @@ linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x,
   asm("" : "+s"(minus1));
   float scale[AN];
   scale[0] = scale[AN - 1] = kScale;
+  if (threadIdx.x == 0) again = 0;
   if (threadIdx.x < AN * 16) {
     row_max[threadIdx.x] = 0;
     row_inv[threadIdx.x] = 1.f / kScale;
   }
+  float wmax[AN];
+  wmax[0] = wmax[AN - 1] = 0.f;
   float4v acc[AN][CT];
   auto run = [&](auto careful) {
-    float wmax = 0.f;
+    constexpr bool kCareful = decltype(careful)::value;
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
@@ -395,34 +403,39 @@ linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x,
       for (int a = 0; a < AN; ++a)
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          split8<decltype(careful)::value>(wv[a][2 * u], wv[a][2 * u + 1], scale[a], hi[a][u], lo[a][u], wmax, minus1);
+          split8<kCareful>(wv[a][2 * u], wv[a][2 * u + 1], scale[a], hi[a][u], lo[a][u], wmax[a], minus1);
       kb += W * 128;
       if (kb < p.k) fetch(kb);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-          const half8 xf = __builtin_bit_cast(half8, xv[c][u]);
+          const half8 xf = __builtin_bit_cast(half8, xv[c][u]), xl = kCareful ? finite8(xf) : xf;
 #pragma unroll
           for (int a = 0; a < AN; ++a) {
             acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[a][u], xf, acc[a][c], 0, 0, 0);
-            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[a][u], xf, acc[a][c], 0, 0, 0);
+            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[a][u], xl, acc[a][c], 0, 0, 0);
           }
         }
     }
-    return block_max(wmax, red, W);
   };
-  if (!scale_ok(run(std::false_type{}))) {
+  run(std::false_type{});
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a sum is infinite or NaN
 #pragma unroll
-    for (int a = 0; a < AN; ++a) {
-      float m = 0.f;
-      for (int kb = wave * 128; kb < p.k; kb += W * 128)
-        for (int u = 0; u < 8; u += 2)
-          m = max8(m, *reinterpret_cast<const float4v*>(wp[a] + kb + 4 * u),
-                   *reinterpret_cast<const float4v*>(wp[a] + kb + 4 * u + 4));
-      atomicMax(&row_max[a * 16 + col], __builtin_bit_cast(int, m));  // m >= 0: ordered as its bits
-    }
-    __syncthreads();
+  for (int a = 0; a < AN; ++a)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) zero[i] = fmaf(acc[a][c][i], 0.f, zero[i]);
+  __syncthreads();  // row_max and again hold their first values
+#pragma unroll
+  for (int a = 0; a < AN; ++a)
+    atomicMax(&row_max[a * 16 + col], __builtin_bit_cast(int, wmax[a]));  // wmax >= 0: ordered as its bits
+  if ((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f) again = 1;
+  __syncthreads();
+  if (threadIdx.x < AN * 16 && !scale_ok(__builtin_bit_cast(float, row_max[threadIdx.x]))) again = 1;
+  __syncthreads();
+  if (again) {  // block-uniform
 #pragma unroll
     for (int a = 0; a < AN; ++a) {
       scale[a] = scale_for(__builtin_bit_cast(float, row_max[a * 16 + col]));
@@ -457,7 +470,7 @@ linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x,
 // MFMAs (156 us; 228 us before the loads ran two stages ahead and the row tiles
 // of a panel shared an XCD).
 template <int MODE, int AN, int CT, int kBK>
-__global__ void __launch_bounds__(512, 2)
+__global__ void __launch_bounds__(512, AN == 1 && kBK == 32 ? 4 : 2)
 linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, int rows, int row_tiles, int panels) {
   constexpr int kG = 2, TN = AN * 64, TS = CT * 64, kRow = kBK / 8;
   constexpr int kWv = TN * kRow, kXv = TS * kRow;                    // 16-byte units of a plane of W, of X
@@ -466,7 +479,7 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
   constexpr int kXS = CT == 4 ? 1 : 2;
   constexpr int kWL = TN * kBK / 8 / 256, kXL = TS * kBK / 8 / 256;  // 8-element units a thread stages
   __shared__ uint4v smem[kG * 2 * kStage];
-  __shared__ float red[8];
+  __shared__ int again;
   __shared__ int row_max[TN];
   __shared__ float row_inv[TN];
   static_assert(sizeof(smem) >= 256 * 16 * AN * CT * 4, "the groups' sums fit the staging buffers");
@@ -504,15 +517,19 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
   float scale[kWL];
 #pragma unroll
   for (int u = 0; u < kWL; ++u) scale[u] = kScale;
+  if (threadIdx.x == 0) again = 0;
   if (threadIdx.x < TN) {
     row_max[threadIdx.x] = 0;
     row_inv[threadIdx.x] = 1.f / kScale;
   }
+  float wmax[kWL];
+#pragma unroll
+  for (int u = 0; u < kWL; ++u) wmax[u] = 0.f;
   float16v acc[AN][CT];
   const int iters = p.k / (kBK * kG);  // the launch takes a kBK that divides k evenly
 
   auto run = [&](auto careful) {
-    float wmax = 0.f;
+    constexpr bool kCareful = decltype(careful)::value;
 #pragma unroll
     for (int a = 0; a < AN; ++a)
 #pragma unroll
@@ -551,7 +568,10 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
       for (int u = 0; u < kWL; ++u) {
         const int i = at((u * 256 + tid) / kRow, tid % kRow);
         half8 hi, lo;
-        split8<decltype(careful)::value>(wv[R][u][0], wv[R][u][1], scale[u], hi, lo, wmax, minus1);
+        split8<kCareful>(wv[R][u][0], wv[R][u][1], scale[u], hi, lo, wmax[u], minus1);
+        // the units in turn: left to interleave their maxima, the compiler waits for LDS more
+        // often (gate and up, 1,024 rows: 151 -> 145 us; 128 rows: 37.4 -> 34.3)
+        if (!kCareful && u + 1 < kWL) asm("" : "+v"(wmax[u + 1]), "+v"(wv[R][u + 1][0]) : "v"(wmax[u]));
         s[i] = __builtin_bit_cast(uint4v, hi);
         s[kWv + i] = __builtin_bit_cast(uint4v, lo);
       }
@@ -574,7 +594,8 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
 #pragma unroll
           for (int c = 0; c < CT; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, xf[c], acc[a][c], 0, 0, 0);
 #pragma unroll
-          for (int c = 0; c < CT; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, xf[c], acc[a][c], 0, 0, 0);
+          for (int c = 0; c < CT; ++c)
+            acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, kCareful ? finite8(xf[c]) : xf[c], acc[a][c], 0, 0, 0);
         }
       }
     };
@@ -599,17 +620,23 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
       __syncthreads();
     }
     if (it < iters) products(even);
-    return block_max(wmax, red, 8);
   };
-  if (!scale_ok(run(std::false_type{}))) {
+  run(std::false_type{});
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a sum is infinite or NaN
 #pragma unroll
-    for (int u = 0; u < kWL; ++u) {
-      float m = 0.f;
-      for (int kb = grp * kBK + kc; kb < p.k; kb += kG * kBK)
-        m = max8(m, *reinterpret_cast<const float4v*>(wrow[u] + kb), *reinterpret_cast<const float4v*>(wrow[u] + kb + 4));
-      atomicMax(&row_max[(u * 256 + tid) / kRow], __builtin_bit_cast(int, m));  // m >= 0: ordered as its bits
-    }
-    __syncthreads();
+  for (int a = 0; a < AN; ++a)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) zero[i & 3] = fmaf(acc[a][c][i], 0.f, zero[i & 3]);
+#pragma unroll
+  for (int u = 0; u < kWL; ++u)  // wmax >= 0: ordered as its bits
+    atomicMax(&row_max[(u * 256 + tid) / kRow], __builtin_bit_cast(int, wmax[u]));
+  if ((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f) again = 1;
+  __syncthreads();
+  if (threadIdx.x < TN && !scale_ok(__builtin_bit_cast(float, row_max[threadIdx.x]))) again = 1;
+  __syncthreads();
+  if (again) {  // block-uniform
 #pragma unroll
     for (int u = 0; u < kWL; ++u) {
       const int r = (u * 256 + tid) / kRow;
@@ -617,6 +644,7 @@ linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, 
       row_inv[r] = 1.f / scale[u];  // the row's threads agree
     }
     run(std::true_type{});
+    __syncthreads();
   }
   float* m = reinterpret_cast<float*>(smem) + wave * AN * CT * 16 * 64 + lane;
   if (grp == 1) {

@@ -21,7 +21,8 @@
 // deviation 1 to 16); attention.hip's fp32 products of fp32 weights are off by
 // 3.2e-7 to 1.6e-6 on the same inputs.
 // Infinities in V: hi * V and lo * V cancel or meet 0 where p * V is infinite, so
-// a block that finds a NaN in its sums takes its rows again in fp32 (careful_row).
+// a block that finds a sum that is not finite takes its rows again in fp32
+// (careful_row).
 // The maximum is moved only when a lane's sum of p says that it must be, which
 // takes the max scan and its cross-lane step out of most tiles.
 //
@@ -289,13 +290,13 @@ prompt_attn_kernel(const uint16_t* __restrict__ q, int B, int Hq, int G, const u
     __syncthreads();
   }
 
-  bool nan = false;
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};  // NaN where a sum is infinite or NaN
 #pragma unroll
   for (int d = 0; d < kDT; ++d)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) nan = nan || o[d][i] != o[d][i];
-  nan = __any(nan);
-  if (lane == 0) s_hi[wave] = nan;  // its bounds were read before the barriers above
+    for (int i = 0; i < 16; ++i) zero[i & 3] = fmaf(o[d][i], 0.f, zero[i & 3]);
+  const int odd = __any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f);
+  if (lane == 0) s_hi[wave] = odd;  // its bounds were read before the barriers above
   __syncthreads();
   int any = s_hi[0];
 #pragma unroll

@@ -229,7 +229,10 @@ int rfsn_dense_attention(const void* q_dev, int32_t B, int32_t Hq, int32_t D,
  *  - mode 1 (SwiGLU, n_0 == n_1): out_0 = fp16(act * up), up = fp16(x W_1^T),
  *    act = fp16(g * sigmoid(g)), g = fp16(x W_0^T).
  *  - mode 2: out_0 = fp16(residual + fp16(x W_0^T)), residual [rows][n_0].
- * Sums are fp32; weights keep their fp32 value to 23 bits or 2^-37.
+ * Sums are fp32.  For one row of x weights are exact.  For more, a weight keeps
+ * its value to 2^-23 of itself or 2^-37, whichever is more; where a weight row's
+ * largest value W is past 15.9 or below 2^-12, to 2^-23 of itself or 2^-39 W.
+ * Infinite and NaN values of x and W give the infinities and NaN of fp32 sums.
  * k a multiple of 64 up to 32768, n_t multiples of 4 (of head_dim with rotary
  * embedding), buffers 16-byte aligned. */
 typedef struct rfsn_linear_params {

@@ -348,3 +348,16 @@ def test_llama_layer_saved_without_shapes(device, tmp_path):
     old.__setstate__(state)
     x = torch.from_numpy(randn16(rng(39), 1, 9, 512)).to(device)
     assert old._shapes == layer._shapes and torch.equal(old(x), layer(x))
+
+
+def test_llama_layer_carries_infinite_and_nan_tokens(device, tmp_path):
+    """A prompt token that is no number reaches itself and the tokens after it, and none before."""
+    layer = _llama(device, tmp_path)
+    x = torch.from_numpy(randn16(rng(40), 1, 90, 512)).to(device)
+    plain = layer(x)
+    for value in (float("nan"), float("inf")):
+        y = x.clone()
+        y[0, 50, 3] = value
+        out = layer(y)
+        assert (out[0, :50] - plain[0, :50]).abs().max() <= 4e-3  # blocks that repeat their sums round anew
+        assert bool(out[0, 50:].isnan().all())  # the norm of an infinite row holds inf * 0

@@ -1,8 +1,8 @@
 """``rfsn_layer_linear`` against float64: one row, the streamed rows (up to 64) and the tiles (past 64), at the
 edges of their row, output and k ranges.
 
-A plain result is one fp16 rounding (2^-11 |y|) of fp32 sums of k products with weights kept to 2^-23: bounded
-by 2^-20 sum |x w| for the k here.  Behind it each fp16 cast point may add 2^-11 of its value once more."""
+A plain result is one fp16 rounding (2^-11 |y|) of fp32 sums of k products with weights kept to 2^-23 (and to
+2^-37, or 2^-39 of their row's largest): bounded by 2^-20 sum |x w| for the k here.  Behind it each fp16 cast point may add 2^-11 of its value once more."""
 
 import numpy as np
 import pytest
@@ -110,6 +110,76 @@ def test_weights_outside_the_first_scale(device, rows):
     assert np.all(np.isinf(o[:, 9]) | (x[:, 9] == 0))
     ok = np.abs(o - y) <= np.abs(y) * 2.0 ** -11 + mag * 2.0 ** -20 + small + 2.0 ** -25
     assert np.all(np.delete(ok, 9, 1))
+
+
+@pytest.mark.parametrize("rows", [1, 5, 20, 50, 90, 300])
+@pytest.mark.parametrize("k", [192, 256])
+def test_small_weights(device, rows, k):
+    """Rows of small weights (all of a matrix, or single rows among ordinary ones) keep their precision."""
+    from apple_amd import kernels as K
+
+    g, x, w = _data(rows, k, 128, rows + k)
+    x = (x.astype(np.float32) * 4096).astype(np.float16)
+    small, mixed = w[0] * np.float32(2.0 ** -26), w[1].copy()
+    mixed[::5] *= np.float32(2.0 ** -26)
+    mixed[7], mixed[8] = 0, small[8] * np.float32(2.0 ** -90)
+    mixed[9, 0] = 5e-5  # the largest of a row of 2^-26
+    x64 = x.astype(np.float64)
+    for m in (small, mixed):
+        o, = K.layer_linear(_t(x, device), [_t(m, device)])
+        y, mag = x64 @ m.T.astype(np.float64), np.abs(x64) @ np.abs(m.T.astype(np.float64))
+        row = np.abs(x64).sum(-1, keepdims=True) * np.abs(m).max(-1)[None] * 2.0 ** -38  # 2^-39, rounded twice
+        f = np.abs(y) < 65000  # the ordinary rows' sums may leave fp16's range
+        assert np.all(np.abs(o.double().cpu().numpy() - y)[f] <= (np.abs(y) * 2.0 ** -11 + mag * 2.0 ** -20 + row + 2.0 ** -25)[f])
+
+
+def _ieee(x, w):
+    """x w^T in float64 with the infinities and NaN of a float32 sum: what meets each product, in any order."""
+    fin = np.where(np.isfinite(x), x, 0).astype(np.float64)
+    y = fin @ w.T.astype(np.float64)
+    inf = np.where(np.isinf(x), np.sign(np.where(np.isinf(x), x, 0)), 0).astype(np.float64)
+    up = np.maximum(inf, 0) @ np.maximum(w, 0).T + np.maximum(-inf, 0) @ np.maximum(-w, 0).T
+    down = np.maximum(inf, 0) @ np.maximum(-w, 0).T + np.maximum(-inf, 0) @ np.maximum(w, 0).T
+    nan = np.isnan(x).any(-1, keepdims=True) | (np.isinf(x).astype(np.float64) @ (w == 0).T.astype(np.float64) > 0)
+    y[up > 0], y[down > 0] = np.inf, -np.inf
+    y[nan | ((up > 0) & (down > 0))] = np.nan
+    return y
+
+
+@pytest.mark.parametrize("rows", [1, 2, 20, 50, 70, 300])
+@pytest.mark.parametrize("k,n", [(192, 128), (256, 128), (256, 4100)])
+def test_infinite_inputs(device, rows, k, n):
+    """An infinite x is infinite in every output its weights lead to, whether a weight has a low half or not, down to
+    the smallest; two of opposite sign, or one that meets a weight of 0, give NaN; other rows are untouched."""
+    from apple_amd import kernels as K
+
+    g, x, w = _data(rows, k, n, rows * k + n)
+    m = w[0].copy()
+    m[::3] = m[::3].astype(np.float16)          # no low half
+    m[5, 100], m[6, 100], m[7, 100] = 0.0, 2.0 ** -60, -(2.0 ** -60)
+    m[1::7, 30] = np.abs(m[1::7, 30])
+    plain = x.astype(np.float64) @ m.T.astype(np.float64)
+    x[0, 100] = np.inf
+    if rows > 1:
+        x[rows - 1, 30], x[rows - 1, 31] = -np.inf, np.inf
+    if rows > 20:
+        x[17, 3], x[18, 64] = np.nan, -np.inf
+    want = _ieee(x, m)
+    res = np.ones((rows, n), np.float16)
+    for o, add in ((K.layer_linear(_t(x, device), [_t(m, device)])[0], 0.0),
+                   (K.layer_linear(_t(x, device), [_t(m, device)], K.LINEAR_RESIDUAL, residual=_t(res, device))[0], 1.0)):
+        o = o.double().cpu().numpy()
+        assert np.array_equal(np.isnan(o), np.isnan(want)) and np.array_equal(o[np.isinf(want)], want[np.isinf(want)])
+        f = np.isfinite(want)
+        assert np.all(np.abs(o[f] - want[f] - add) <= (np.abs(want[f]) + add) * 2.0 ** -10 + 2.0 ** -12)
+    # SwiGLU of the same: gate and up past the norm's infinities (none here) as their products make them
+    act, = K.layer_linear(_t(x, device), [_t(m, device), _t(w[1], device)], K.LINEAR_SWIGLU)
+    act = act.double().cpu().numpy()
+    with np.errstate(all="ignore"):
+        gate, up = want, _ieee(x, w[1])
+        ref = (gate * (1 / (1 + np.exp(-gate)))) * up
+    assert np.array_equal(np.isnan(act), np.isnan(ref))
+    assert np.array_equal(act[np.isinf(ref)], ref[np.isinf(ref)])
 
 
 @pytest.mark.parametrize("k", [64, 192, 320, 2048, 2112, 8192, 8256, 32768])
