@@ -40,6 +40,9 @@ from .storage import AsyncHierarchicalRouterMLX, RFSNConfig
 
 MASK_FILL_VALUE = -1e30
 
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+_wrapped = torch._C._functorch.is_functorch_wrapped_tensor  # a tensor that torch.func maps or differentiates
+
 _INV_FREQ_LOCK = threading.Lock()  # two calls that miss a layer's kept frequencies make them once
 
 
@@ -99,19 +102,18 @@ def _unwatched(x: torch.Tensor) -> bool:
     intercepts its operators or casts them, and it is a plain tensor (or
     parameter).  A tensor that torch.func maps or differentiates has a plain
     type and no address: it is told by its wrapper, before anything reads it."""
-    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
+    return (type(x) in _PLAIN_TYPES and not (x.requires_grad and torch.is_grad_enabled())
             and not torch.is_autocast_enabled() and not torch.compiler.is_compiling()
             and torch._C._get_tracing_state() is None and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._len_torch_function_stack() == 0 and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._functorch.is_functorch_wrapped_tensor(x))
+            and not _wrapped(x))
 
 
 def _plain_weight(w: torch.Tensor, device: torch.device) -> bool:
     """A weight the projection kernel reads as it is: fp32, contiguous, aligned, on the device, and nothing
     watches it (``_unwatched``, whose checks of the call itself the caller has made for its input)."""
-    return (type(w) in (torch.nn.Parameter, torch.Tensor) and not torch._C._functorch.is_functorch_wrapped_tensor(w)
-            and not (w.requires_grad and torch.is_grad_enabled()) and w.dtype is torch.float32 and w.device == device
-            and w.is_contiguous() and w.data_ptr() % 16 == 0)
+    return (type(w) in _PLAIN_TYPES and not _wrapped(w) and not (w.requires_grad and torch.is_grad_enabled())
+            and w.dtype is torch.float32 and w.device == device and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
 class RFSNDecoderLayerMLX(torch.nn.Module):
@@ -305,7 +307,7 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         if self.device.type == "cuda":
             self._inv_freq()
         self.rotary_module = rotary_module
-        shapes = self._shapes = self._weight_shapes(intermediate_size)
+        shapes = self._set_shapes(intermediate_size)
         g = generator if generator is not None else torch.Generator().manual_seed(4321 + layer_idx)
         for name in self.WEIGHTS:
             if weights is not None:
@@ -322,12 +324,16 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         self.disk_cache_dir = Path(config.disk_cache_dir) / f"llama_layer_{layer_idx}"
         self.cache = RFSNv10KVCacheMLX(config, layer_idx=layer_idx, device=self.device)
 
-    def _weight_shapes(self, inter: int) -> Dict[str, torch.Size]:
+    def _set_shapes(self, inter: int) -> Dict[str, torch.Size]:
+        """The weights' shapes, and whether ``rfsn_layer_linear`` takes projections of them."""
         D, qd, kvd = self.hidden_dim, self.num_heads * self.head_dim, self.num_kv_heads * self.head_dim
         shapes = {"input_layernorm": (D,), "post_attention_layernorm": (D,), "q_proj": (qd, D), "k_proj": (kvd, D),
                   "v_proj": (kvd, D), "o_proj": (D, qd), "gate_proj": (inter, D), "up_proj": (inter, D),
                   "down_proj": (D, inter)}
-        return {n: torch.Size(s) for n, s in shapes.items()}
+        self._shapes = {n: torch.Size(s) for n, s in shapes.items()}
+        self._linear_ok = (K.layer_linear_ok(D, (qd + 2 * kvd,), self.head_dim) and K.layer_linear_ok(D, (inter, inter))
+                           and K.layer_linear_ok(qd, (D,)) and K.layer_linear_ok(inter, (D,)))
+        return self._shapes
 
     @property
     def cache_tokens(self) -> int:
@@ -373,18 +379,17 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         """Whether ``rfsn_layer_linear`` runs this call's projections: a plain
         [1, S, hidden] fp16 input and rotary tables nothing watches, weights
         as it reads them."""
-        D, qkv = self.hidden_dim, (self.num_heads + 2 * self.num_kv_heads) * self.head_dim
-        if (not _unwatched(h16) or h16.dim() != 3 or h16.shape[1] == 0 or int(h16.shape[2]) != D or not h16.is_cuda
+        if (not self._linear_ok or not _unwatched(h16) or h16.dim() != 3 or h16.shape[1] == 0
+                or int(h16.shape[2]) != self.hidden_dim or not h16.is_cuda
                 or h16.device.index != torch.cuda.current_device()
-                or not all(_unwatched(t) and t.device == h16.device for t in tables or ())):
+                or tables is not None and not all(_unwatched(t) and t.device == h16.device for t in tables)):
             return False
+        device, weights = h16.device, self._parameters
         for name, shape in self._shapes.items():
-            w = self._parameters.get(name)
-            if w is None or w.shape != shape or not _plain_weight(w, h16.device):
+            w = weights.get(name)
+            if w is None or w.shape != shape or not _plain_weight(w, device):
                 return False
-        inter = self._shapes["gate_proj"][0]
-        return (K.layer_linear_ok(D, (qkv, ), self.head_dim) and K.layer_linear_ok(D, (inter, inter))
-                and K.layer_linear_ok(self.num_heads * self.head_dim, (D,)) and K.layer_linear_ok(inter, (D,)))
+        return True
 
     def _rows(self, h16: torch.Tensor) -> torch.Tensor:
         """[1, S, hidden] as the contiguous, aligned rows [S, hidden] the projection kernel reads."""
@@ -438,8 +443,8 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
 
     def __setstate__(self, state):
         super().__setstate__(state)
-        if "_shapes" not in self.__dict__:  # a layer saved before it kept its weights' shapes
-            self._shapes = self._weight_shapes(int(self.down_proj.shape[1]))
+        if "_linear_ok" not in self.__dict__:  # a layer saved before it kept what its weights' shapes allow
+            self._set_shapes(int(self.down_proj.shape[1]))
 
     def _session_step(self, session, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         session.left = None  # a step that raises leaves a launch to rebuild

@@ -342,12 +342,14 @@ def test_llama_layer_saved_without_shapes(device, tmp_path):
     import copy
 
     layer = _llama(device, tmp_path)
-    state = copy.deepcopy(layer.__getstate__())
-    del state["_shapes"]
-    old = type(layer).__new__(type(layer))
-    old.__setstate__(state)
     x = torch.from_numpy(randn16(rng(39), 1, 9, 512)).to(device)
-    assert old._shapes == layer._shapes and torch.equal(old(x), layer(x))
+    for names in (["_shapes", "_linear_ok"], ["_linear_ok"]):
+        state = copy.deepcopy(layer.__getstate__())
+        for n in names:
+            del state[n]
+        old = type(layer).__new__(type(layer))
+        old.__setstate__(state)
+        assert old._shapes == layer._shapes and old._native(x) and torch.equal(old(x), layer(x))
 
 
 def test_llama_layer_carries_infinite_and_nan_tokens(device, tmp_path):
