@@ -937,14 +937,19 @@ def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, token
     as decode-once-then-attend (``decode_ref`` / ``decode``, then the matrix
     cores' ``blockwise_attention``) than decoded in registers per query.
 
-    The exact in-register kernel decodes every K/V vector again for each
-    query, so its time follows queries * tokens * q_heads: past 3e7
-    coordinates from 4 queries on, decoding once wins (D 128, 32 heads, 1,000
-    tokens: 84 -> 57 us at 8 queries; 4,096 tokens, 128 queries: 3,834 -> 71
-    us).  The score tables (``tables``) cost 15 to 27 us per query of 32 heads
-    whatever the window, decoding 3.3 us per 2^20 coordinates whatever the
-    queries: even near queries * q_heads * 2^18 = tokens * kv_heads * D (12,000
-    tokens x 32 heads: 120 against 150 us at 4 queries, 211 against 150 at 8).
+    Decoding once takes at least 57 us (the host's launches), then 35 us and
+    2.0 us per 2^20 window coordinates (tokens * kv_heads * D).  The exact
+    kernel in registers decodes every K/V vector again for each query, once for
+    the query heads that share it: its time follows queries * tokens * D times
+    three quarters of the KV heads and a quarter of the query heads, and passes
+    60 us at 2.0e7 to 2.25e7 of them (4 to 64 queries, 256 to 4,096 tokens, D 64
+    and 128, 32 / 32, 32 / 8 and 8 / 8 heads, gated and subspace formats, each
+    side timed): 8 queries x 1,000 tokens, D 128: 80 -> 61 us at 32 / 32 heads,
+    but 44 against 61 at 32 / 8.  The score tables (``tables``) take about 38 us
+    and 9.5 us per 32 query heads, whatever the window: even near 2^17 window
+    coordinates per query head (4,096 tokens, 32 / 32 heads, D 128: 70 and 70 us
+    at 4 queries; 8,192 tokens: 69 against 99 at 4, 107 against 100 at 8), and
+    below 96 query heads under the other's 57 us.
     The decoded window takes at most ``window_bytes`` for K and V together."""
     if head_dim not in (64, 128) or kv_heads <= 0 or q_heads % kv_heads or q_heads // kv_heads not in (1, 2, 4, 8):
         return False
@@ -952,8 +957,8 @@ def decode_first(queries: int, q_heads: int, kv_heads: int, head_dim: int, token
     if queries < DECODE_FIRST_QUERIES or 4 * window > window_bytes:
         return False
     if tables:
-        return queries * q_heads << 18 >= window
-    return queries * tokens * q_heads * head_dim >= 30_000_000
+        return queries * q_heads >= 96 and queries * q_heads << 17 >= window
+    return queries * tokens * head_dim * (3 * kv_heads + q_heads) >= 4 * 24_000_000
 
 
 def _ref_format_params(k_pq_cb: torch.Tensor, k_rvq_cb: Optional[torch.Tensor], rvq_subspaces: int,
