@@ -1174,7 +1174,8 @@ __global__ void __launch_bounds__(W * 64, 1) warm_encode_fused_kernel(const Enco
 // sixteen: the list is complete if every lane's fourth is apart from the first.
 // 131,072 rows of 128 x 4 stages of 4,096 (550 GFLOP): 880 us -> 623, 0.88 PFLOP/s;
 // 4,000 rows: 510 -> 194.  Left: the four-centroid reads (1 KB of L2 a row and stage),
-// and MFMA, VALU and LDS phases that two waves a SIMD overlap in part only.
+// and MFMA, VALU and LDS phases that two waves a SIMD (one at D 256, whose LDS leaves
+// one block a CU) overlap in part only.
 //
 // Screening: a block (4 waves) holds 4 * kRvqSets * 16 rows; each wave holds
 // kRvqSets B operands of 16 rows as -fp16(x) (v_mfma_f32_16x16x32_f16: lane l
@@ -2292,9 +2293,16 @@ int launch_rvq_mfma(const void* resid, int64_t ld, const int32_t* offsets, int64
                        (const float*)r, (const float*)rmax, run, codes);
     return check_launch("rvq_encode_full");
   }
-  // Sets per wave.  Two blocks run on a CU at a time: 256 blocks of 1, 2 or 4 sets take about
-  // 11, 14, 21 units and 512 of them 14, 19, 31 (2 stages of 4,096, D 128: 109, 121, 198 us at
-  // 4,000 rows; 266, 184, 216 at 65,536; 488, 340, 312 at 131,072): the sets whose rounds cost least.
+  // Sets per wave: those whose rounds of blocks cost least, by the times of 2 stages of 4,096 at
+  // D 128, where two blocks run on a CU at a time: 256 blocks of 1, 2 or 4 sets take about 11, 14,
+  // 21 units and 512 of them 14, 19, 31 (us with 1, 2, 4 sets: 108, 122, 194 at 4,000 rows; 261,
+  // 185, 213 at 65,536; 482, 341, 308 at 131,072).  D 256, whose 82 KB of LDS leave one block a CU
+  // (148, 213 us at 4,000 rows; 291, 227 at 32,768; 1,045, 803 at 131,072), and other codebooks
+  // fall the same way: timed at D 64, 128 and 256, 256 to 4,096 centroids and 500 to 131,072 rows
+  // the choice is within 4 % of the best, but for 16,385 to 40,000 rows at D 64 or of at most
+  // 1,024 centroids, where 1 set is 2 to 20 % faster than the 2 taken (D 128, 256 centroids,
+  // 24,000 rows: 36 against 43 us; by keys, 57), and 10 % at D 256 with 256 centroids and 40,000
+  // rows or D 128 with 1,024 and 98,304.
   int sets = 1;
   int64_t least = INT64_MAX;
   const auto consider = [&](int n, int one, int two) {
@@ -2338,7 +2346,9 @@ int launch_warm_encode_fused(const rfsn_format* f, EncodeJobs& jobs, hipStream_t
   // Waves per block.  A block's tables take most of a CU's LDS, so blocks run 256 at
   // a time, and such a round costs about 15 + 1.75 W us (4, 8, 16 waves: 22, 28, 43
   // us at M 8 + RVQ 8 + top-4): the W whose rounds cost least.  32,768 vectors: 28
-  // us in 256 blocks of 8 waves, 43 in 128 of 16.
+  // us in 256 blocks of 8 waves, 43 in 128 of 16.  Timed for M 8 and 16, with and
+  // without the RVQ and the top-4 stage, 256 to 262,144 vectors, the choice is within
+  // 7 % of the best, but for 40,000 vectors of M 8 PQ alone (22 against 19 us with 4 waves).
   int W = 16, blocks = 0;
   int64_t least = INT64_MAX;
   for (int w = 16; w >= 4; w /= 2) {
