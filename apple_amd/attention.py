@@ -109,12 +109,12 @@ class RFSNHybridAttentionMLX:
         T = key_store.num_tokens
         if T == 0:
             return torch.zeros_like(q)
-        dev = quantizer.device
+        dev = torch.device(quantizer.device)
         kst = _on(key_store, dev)
         vst = _on(value_store, dev)
         pos = _normalize_query_positions(query_positions, B, Hq, T - 1, dev) if causal else None
         cb, rcb = quantizer.pq.codebooks, quantizer.rvq_codebooks
-        f = quantizer.warm_format()
+        f = quantizer.warm_format() if quantizer.subspace else None
         # score tables with their drift guard (config.score_table_tolerance)
         # for decode-sized calls of the reference format over enough coded
         # tokens for the tables to beat the exact decode
@@ -142,8 +142,8 @@ class RFSNHybridAttentionMLX:
         out = K.ref_attention(q.to(device=dev, dtype=torch.float16), kv_heads=key_store.num_heads,
                               scale=self.scale, causal=causal, qpos=pos,
                               segments=[K.ref_store_segment(kst, vst, 0, T, 0, head_major=hm)], k_pq_cb=cb, v_pq_cb=cb,
-                              k_rvq_cb=rcb, v_rvq_cb=rcb, rvq_subspaces=f.rvq_subspaces if quantizer.subspace else 0,
-                              sparse_k=f.sparse_k if quantizer.subspace else 0, **tables)
+                              k_rvq_cb=rcb, v_rvq_cb=rcb, rvq_subspaces=f.rvq_subspaces if f is not None else 0,
+                              sparse_k=f.sparse_k if f is not None else 0, **tables)
         return out.to(q.dtype)
 
     def _table_stats(self, quantizer: HybridQuantizerMLX) -> torch.Tensor:
@@ -159,8 +159,8 @@ class RFSNHybridAttentionMLX:
         return memo[1]
 
 
-def _on(store: CompressedTensorMLX, device) -> CompressedTensorMLX:
-    if store.pq_codes.device == torch.device(device):
+def _on(store: CompressedTensorMLX, device: torch.device) -> CompressedTensorMLX:
+    if store.pq_codes.device == device:
         return store
     d = lambda t: None if t is None else t.to(device)
     return CompressedTensorMLX(d(store.pq_codes), d(store.rvq_codes), d(store.rvq_mask), d(store.rvq_offsets),
