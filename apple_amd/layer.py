@@ -422,11 +422,12 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         (``DecodeSession``: most steps re-issue one prepared launch, which
         appends the token itself), or None where the general ``update`` +
         ``attention_forward`` has to run: a cold tier, or a step that may spill
-        into one, another tier policy, or a format the fused kernel does not
-        serve.  A cache that was written, reconfigured or recalibrated since
+        into one, another tier policy, a format the fused kernel does not
+        serve, or a cache class of the caller's (whose methods a session would
+        pass by).  A cache that was written, reconfigured or recalibrated since
         the session's last step has its launch built anew."""
         c = self.cache
-        if (not c._recency or not c._subspace or c.num_cold or c._kq is None or c.hot_capacity < 2 * c.HOT_BLOCK
+        if (type(c) is not RFSNv10KVCacheMLX or not c._recency or not c._subspace or c.num_cold or c._kq is None or c.hot_capacity < 2 * c.HOT_BLOCK
                 or c.num_warm + c.HOT_BLOCK > c.warm_capacity or not c._fused_ok(self.num_heads)):
             return None
         s = getattr(self, "_decode", None)

@@ -363,3 +363,27 @@ def test_llama_layer_carries_infinite_and_nan_tokens(device, tmp_path):
         out = layer(y)
         assert (out[0, :50] - plain[0, :50]).abs().max() <= 4e-3  # blocks that repeat their sums round anew
         assert bool(out[0, 50:].isnan().all())  # the norm of an infinite row holds inf * 0
+
+
+def test_llama_layer_calls_the_methods_of_its_cache(device, tmp_path):
+    """A cache class of the caller's sees every cached step through its own methods."""
+    from apple_amd.cache import RFSNv10KVCacheMLX
+
+    calls = []
+
+    class Counted(RFSNv10KVCacheMLX):
+        def update(self, *a, **kw):
+            calls.append("update")
+            return super().update(*a, **kw)
+
+        def attention_forward(self, *a, **kw):
+            calls.append("attend")
+            return super().attention_forward(*a, **kw)
+
+    layer = _llama(device, tmp_path)
+    layer.cache = Counted(layer.config, layer_idx=0, device=device)
+    g = rng(41)
+    layer.prefill_cache(torch.from_numpy(randn16(g, 1, 70, 512)).to(device), reset=False)
+    for _ in range(3):
+        layer(torch.from_numpy(randn16(g, 1, 1, 512)).to(device), use_cache=True)
+    assert calls == ["update"] + ["update", "attend"] * 3
