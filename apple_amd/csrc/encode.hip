@@ -1172,7 +1172,8 @@ __global__ void __launch_bounds__(W * 64, 1) warm_encode_fused_kernel(const Enco
 // from the unrounded x, a wave per row, and what that leaves open (2E' = 2.5 (mfma
 // + canon)) the float64 chain.  A lane keeps four keys and the row merges its lanes'
 // sixteen: the list is complete if every lane's fourth is apart from the first.
-// 131,072 rows of 128 x 4 stages of 4,096 (550 GFLOP): 880 us -> 623, 0.88 PFLOP/s;
+// 131,072 rows of 128 x 4 stages of 4,096 (550 GFLOP): 880 us -> 626, 0.88 PFLOP/s
+// (matrix cores busy 41 %, VALU issue 43 %, LDS 20 %, waves waiting 32 %);
 // 4,000 rows: 510 -> 194.  Left: the four-centroid reads (1 KB of L2 a row and stage),
 // and MFMA, VALU and LDS phases that two waves a SIMD (one at D 256, whose LDS leaves
 // one block a CU) overlap in part only.

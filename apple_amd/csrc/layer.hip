@@ -21,8 +21,10 @@
 //
 // The Llama-3.2-1B layer's seven matrices (243 MB of fp32), torch's fp32 products
 // against this file, without the elementwise kernels around the former:
-//   1 row      88 -> 54 us (4.5 TB/s; gate and up 5.4 TB/s)
-//   1,024 rows 865 -> 317 us (393 TFLOP/s of fp32 products)
+//   1 row      88 -> 50 us (4.8 TB/s; passes in a row find half of the weights in
+//              the 256 MB last-level cache: 120 MB come from HBM)
+//   1,024 rows 865 -> 298 us (418 TFLOP/s of fp32 products) on their own in a row,
+//              345 us in the layer's pass under a kernel trace
 #include "rfsn_common.h"
 #include "rfsn_internal.h"
 
@@ -465,10 +467,11 @@ linear_skinny_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x,
 // rows under SwiGLU), two groups of 4 waves that take k runs of 32 in turn (an
 // in-block split of k: with one block or two per CU every SIMD then has two
 // waves or more), W split into its hi and lo planes on its way to LDS.
-// Bound: the LDS reads that feed the MFMAs (two per product), which take about as
-// long as these at AN 2, CT 2; gate and up at 1,024 rows 880 TFLOP/s of issued
-// MFMAs (156 us; 228 us before the loads ran two stages ahead and the row tiles
-// of a panel shared an XCD).
+// No unit is full: at 1,024 rows the matrix cores are busy 39, 42 and 50 % of the
+// cycles (q, k and v; down; gate and up), VALU issue 30 %, LDS 32, 43 and 28 %, and
+// a SIMD's two waves wait 27 to 36 % of theirs between the barriers.  Gate and up
+// run at 830 to 950 TFLOP/s of issued MFMAs (145 to 166 us by box and clock; 228 us
+// before the loads ran two stages ahead and the row tiles of a panel shared an XCD).
 template <int MODE, int AN, int CT, int kBK>
 __global__ void __launch_bounds__(512, AN == 1 && kBK == 32 ? 4 : 2)
 linear_tiles_kernel(const rfsn_linear_params p, const uint16_t* __restrict__ x, int rows, int row_tiles, int panels) {
