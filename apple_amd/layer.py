@@ -302,10 +302,10 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
         self.rms_norm_eps = rms_norm_eps
         self.rope_theta = rope_theta
         self.rope_scaling = dict(rope_scaling) if rope_scaling else None
-        if self.rope_scaling:
-            rope_inv_freq(config.head_dim, rope_theta, self.rope_scaling)  # rejects unsupported types now
         if self.device.type == "cuda":
-            self._inv_freq()
+            self._inv_freq()  # rejects unsupported scaling types now
+        elif self.rope_scaling:
+            rope_inv_freq(config.head_dim, rope_theta, self.rope_scaling)
         self.rotary_module = rotary_module
         shapes = self._set_shapes(intermediate_size)
         g = generator if generator is not None else torch.Generator().manual_seed(4321 + layer_idx)
@@ -398,21 +398,19 @@ class Llama32DecoderLayerMLX(torch.nn.Module):
 
     def _inv_freq(self) -> torch.Tensor:
         """``rope_inv_freq`` on the device, kept for the layer's present rotary settings.  Calls on any stream read
-        it, so its stream is waited for once, where it is made (at construction, for the first settings), and the
-        device before one of other settings is dropped.  Inside a graph capture, where nothing may be waited for
-        and what is made holds nothing before the replay, a missing one is made for the call alone."""
+        it: it is copied from host memory, which is done when the copy returns, at construction for the first
+        settings; before one of other settings is dropped the device is waited for.  Inside a graph capture, which
+        allows neither, a missing one is made on the device for the call alone."""
         key = (self.head_dim, self.rope_theta, None if not self.rope_scaling else dict(self.rope_scaling))
         kept = self.__dict__.get("_inv_freq_kept")
         if kept is None or kept[0] != key:
+            if torch.cuda.is_current_stream_capturing():
+                return rope_inv_freq(*key, self.device).contiguous()
             with _INV_FREQ_LOCK:
                 kept = self.__dict__.get("_inv_freq_kept")
                 if kept is None or kept[0] != key:
-                    made = (key, rope_inv_freq(*key, self.device).contiguous())
-                    if torch.cuda.is_current_stream_capturing():
-                        return made[1]
-                    if kept is None:
-                        torch.cuda.current_stream(self.device).synchronize()
-                    else:
+                    made = (key, rope_inv_freq(*key, torch.device("cpu")).to(self.device))
+                    if kept is not None:
                         torch.cuda.synchronize(self.device)
                     self._inv_freq_kept = kept = made
         return kept[1]
