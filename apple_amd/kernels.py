@@ -302,17 +302,19 @@ def blockwise_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tenso
     out = torch.empty_like(q)
     qp = None if qpos is None else _qpos(qpos, B, Hq, q.device)
     lib = L.load()
-    # partials of the splits a launch may choose: enough blocks to fill the
-    # chip, so few once there are many query rows
-    rows = B * max(1, Hq // max(Hkv, 1))
-    heads = max(Hkv, 1)  # sizes of 0 are the launch's to refuse
-    splits_max = max(1, min(1024, -(-T // 256), max(-(-1024 // max(B * heads, 1)),
-                                                    -(-512 // (heads * max(-(-rows // 256), 1))))))
+    # partials of the splits a launch may choose, of at least 256 tokens: with
+    # many query rows few, enough to fill the chip (sizes of 0 are the launch's
+    # to refuse)
+    splits_max = min(1024, (T + 255) >> 8) or 1
+    if B > 1 and splits_max > 1:
+        heads = max(Hkv, 1)
+        rows = B * max(1, Hq // heads)
+        splits_max = min(splits_max, max(-(-1024 // (B * heads)), -(-512 // (heads * -(-rows // 256)))))
     wsb = lib.rfsn_attention_workspace_bytes(B, Hq, D, splits_max)
     ws = torch.empty(wsb, dtype=torch.uint8, device=q.device)
     L.call("rfsn_dense_attention" if dense else "rfsn_blockwise_attention", q.data_ptr(), B, Hq, D,
-           keys.data_ptr() if T else None, values.data_ptr() if T else None, T, Hkv, keys.stride(0), keys.stride(1), float(scale), int(causal),
-           L.ptr(qp), out.data_ptr(), ws.data_ptr(), wsb, _stream(q))
+           keys.data_ptr() if T else None, values.data_ptr() if T else None, T, Hkv, keys.stride(0), keys.stride(1),
+           float(scale), int(causal), L.ptr(qp), out.data_ptr(), ws.data_ptr(), wsb, _stream(q))
     return out
 
 
